@@ -228,6 +228,13 @@ int64_t moe_prefill_route_stats_offset(int tokens, int width, int ff, int expert
 // strata_norm mode 0 (scale 1) over `rows` rows of `cols`, on the context's stream.
 int norm_launch(sm_ctx *ctx, const float *X, const float *gamma, float *Y, int cols, int rows, float eps);
 
+// Dense projections of a token batch (project_batch.hip), bit-identical to
+// the general kernels: bits 16 = bf16 weights, else quantized codes.
+bool project_batch_takes(int bits, int cols, int tokens, uint64_t X, uint64_t codes, int group, int bias, int codebook);
+int project_batch(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets,
+                  float *Y, int cols, int rows, int tokens, int stride, int out, int group, int bias, int codebook,
+                  int has_offset);
+
 // ------------------------------------------------ kernels by name (sm_run)
 // One 64-bit slot per reference parameter: a buffer handle, or the int32 /
 // float32 bit pattern in the low 32 bits.

@@ -1,0 +1,287 @@
+// Dense projections of a token batch (strata_bf16_project and
+// strata_quant_project with two or more tokens): every weight is read and
+// widened once for up to 16 tokens, with the reference's sums.
+//
+// The reference's order (kernels/strata.cu:156-165) is 64 partial sums per
+// output, partial p over the columns p, p + 64, ... one rounded product and
+// one rounded sum at a time, then a tree. The sums have to stay on the vector
+// unit, but the products need not: v_mfma_f32_4x4x1_16b_f32 with a zero
+// accumulator forms 16 independent 4 x 4 outer products, each element one
+// f32 product rounded to nearest even (subnormals kept; an exact -0 becomes
+// +0, which a partial sum that starts at +0 cannot tell apart). A block of
+// the instruction is one column, its rows four tokens and its columns four
+// weight rows, so four of them are the 64 columns of a step and every lane
+// then adds its own 4 x 4 products: one matrix instruction for four vector
+// adds where the vector unit alone would need four multiplies as well.
+//
+// A wave owns four weight rows and 4 NG tokens. Lane l holds columns
+// 4 (l / 4) .. + 3 of the step's 64 for weight row l % 4, and reads the same
+// columns of token 4 g + l % 4 from LDS with one 16-byte load per group of
+// four tokens. The block's four waves share the tokens' columns, which
+// arrive by DMA one chunk of KC steps ahead; the weights go straight to
+// registers one chunk ahead.
+//
+// Bound: vector issue from about 8 tokens (16 tokens: 64 adds and 16 matrix
+// instructions a step; without its loads the kernel takes 26 of its 31 us),
+// the weights' stream below (a load's latency per chunk, 3 TB/s). bf16, 2,560
+// x 10,240 x 16 tokens: 208 -> 31 us, where one wave per output and token
+// read each weight 16 times. Three or four chunks of weights in registers
+// were slower (35 us: fewer waves fit and the loads past the end count).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "internal.h"
+#include "strata_device.h"
+
+using namespace smi;
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void_t;
+
+// The raw weights of one lane and one step: four columns of one row.
+template <int BITS>
+struct Raw {
+    uint32_t code[BITS == 16 ? 2 : 1];
+    float scale, offset;
+};
+
+struct ProjectArgs {
+    const float *X;
+    const uint8_t *codes;
+    const float *scales, *offsets;
+    float *Y;
+    int cols, rows, tokens, stride, out;
+    int group_shift, has_offset;
+    float bias;
+};
+
+// IQ4_NL values (kernels/strata.cu:22-31) as signed bytes, four to a word.
+constexpr uint32_t iq4_word(int a, int b, int c, int d) {
+    return (uint32_t)(a & 255) | (uint32_t)(b & 255) << 8 | (uint32_t)(c & 255) << 16 | (uint32_t)(d & 255) << 24;
+}
+
+template <int BITS>
+__device__ __forceinline__ void load_raw(const ProjectArgs &a, const uint8_t *row_codes, const float *row_scales,
+                                         const float *row_offsets, int col, Raw<BITS> &w) {
+    if (BITS == 16) {
+        const uint2 v = *(const uint2 *)(row_codes + 2 * col);
+        w.code[0] = v.x;
+        w.code[BITS == 16 ? 1 : 0] = v.y;
+    } else {
+        if (BITS == 8) w.code[0] = *(const uint32_t *)(row_codes + col);
+        if (BITS == 4) w.code[0] = *(const uint16_t *)(row_codes + col / 2);
+        if (BITS == 2) w.code[0] = row_codes[col / 4];
+        const int g = col >> a.group_shift;
+        w.scale = row_scales[g];
+        w.offset = row_offsets[g];
+    }
+}
+
+// Widens the four weights in the reference's steps (kernels/strata.cu:168-211).
+// Without offsets +0 is added: that can only turn a weight of -0 into +0, and
+// no partial sum tells a product of -0 from one of +0.
+template <int BITS, bool CODEBOOK>
+__device__ __forceinline__ void widen(const ProjectArgs &a, const Raw<BITS> &w, float (&out)[4]) {
+    if (BITS == 16) {
+        out[0] = __uint_as_float(w.code[0] << 16);
+        out[1] = __uint_as_float(w.code[0] & 0xffff0000u);
+        out[2] = __uint_as_float(w.code[BITS == 16 ? 1 : 0] << 16);
+        out[3] = __uint_as_float(w.code[BITS == 16 ? 1 : 0] & 0xffff0000u);
+        return;
+    }
+    const uint32_t c = w.code[0];
+    if (CODEBOOK) {
+        // the four codes in four bytes, looked up in the table's two halves
+        const uint32_t t = (c | c << 8) & 0x00ff00ffu, b = (t | t << 4) & 0x0f0f0f0fu, s = b & 0x07070707u;
+        const uint32_t lo = __builtin_amdgcn_perm(iq4_word(-49, -35, -22, -10), iq4_word(-127, -104, -83, -65), s);
+        const uint32_t hi = __builtin_amdgcn_perm(iq4_word(53, 69, 89, 113), iq4_word(1, 13, 25, 38), s);
+        const uint32_t m = ((b >> 3) & 0x01010101u) * 255u, v = (hi & m) | (lo & ~m);
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[q] = (float)((int)(v << (24 - 8 * q)) >> 24);
+    } else {
+        // code + bias: both are whole numbers below 2^23, so the f32 sum is exact
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[q] = (float)((c >> (BITS * q)) & ((1u << BITS) - 1u)) + a.bias;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) out[q] = out[q] * w.scale;
+    const float offset = a.has_offset ? w.offset : 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; q++) out[q] = out[q] + offset;
+}
+
+// The reference's tree over columns for one group's 4 x 4 products: partial
+// sums of column 4 b + q are in lanes 4 b .. 4 b + 3 (one weight row each)
+// of p[q], element r for token r. Distances 32, 16, 8 and 4 are lanes 32,
+// 16, 8 and 4 apart; 2 and 1 are q. The two lane swaps leave each row of 16
+// lanes one token: 0, 2, 1, 3.
+__device__ __forceinline__ float tree_columns(const f32x4 (&p)[4]) {
+    float z[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        // (__float_as_uint and back: a bit cast of a vector's element takes its first one)
+        const auto s01 = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[q][0]), __float_as_uint(p[q][1]), false, false);
+        const auto s23 = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[q][2]), __float_as_uint(p[q][3]), false, false);
+        const float u = __uint_as_float(s01[0]) + __uint_as_float(s01[1]);
+        const float v = __uint_as_float(s23[0]) + __uint_as_float(s23[1]);
+        const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(u), __float_as_uint(v), false, false);
+        float w = __uint_as_float(t[0]) + __uint_as_float(t[1]);
+        w = w + sm::dpp_f32<0x108>(0.0f, w);  // row_shl:8
+        z[q] = w + sm::dpp_f32<0x104>(0.0f, w);  // row_shl:4
+    }
+    return (z[0] + z[2]) + (z[1] + z[3]);
+}
+
+// Grid: x = groups of 16 weight rows, y = groups of 4 NG tokens. Rows,
+// tokens and steps past the end read the last valid one and are not stored
+// (a step past the end is not added).
+template <int BITS, bool CODEBOOK, int NG>
+__global__ void __launch_bounds__(256, 2) k_project_batch(ProjectArgs a) {
+    constexpr int KC = 4;  // steps per chunk: one DMA a token
+    constexpr int T = 4 * NG, XS = 64 * KC + 16;  // a token's chunk, padded so that four tokens' reads spread over the banks
+    __shared__ __attribute__((aligned(16))) float s_x[2][T][XS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = lane >> 2, i = lane & 3;
+    const int r0 = blockIdx.x * 16 + wave * 4, t0 = blockIdx.y * T;
+    const int steps = a.cols >> 6, row = min(r0 + i, a.rows - 1);
+    const uint8_t *row_codes = a.codes + (int64_t)row * a.cols * BITS / 8;
+    const int64_t row_groups = BITS == 16 ? 0 : (int64_t)row * (a.cols >> a.group_shift);
+    const float *row_scales = a.scales + row_groups, *row_offsets = (a.has_offset ? a.offsets : a.scales) + row_groups;
+    // Each wave brings every fourth token's chunk: 256 columns, 1 KiB, one DMA.
+    auto stage = [&](int c, int buf) {
+#pragma unroll
+        for (int u = 0; u < NG; u++) {
+            const int t = wave + 4 * u;
+            const float *x = a.X + (int64_t)min(t0 + t, a.tokens - 1) * a.cols;
+            __builtin_amdgcn_global_load_lds(x + min(64 * KC * c + 4 * lane, a.cols - 4), (lds_void_t *)&s_x[buf][t][0], 16,
+                                             0, 0);
+        }
+    };
+    Raw<BITS> cur[KC], next[KC];
+    auto load = [&](int c, Raw<BITS> (&w)[KC]) {
+#pragma unroll
+        for (int k = 0; k < KC; k++)
+            load_raw<BITS>(a, row_codes, row_scales, row_offsets, 64 * min(KC * c + k, steps - 1) + 4 * b, w[k]);
+    };
+    f32x4 acc[NG][4];
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) acc[g][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 xv[2][NG];  // the tokens' columns of this step and of the next
+    auto read_x = [&](int buf, int k) {
+#pragma unroll
+        for (int g = 0; g < NG; g++) xv[k & 1][g] = *(const f32x4 *)&s_x[buf][4 * g + i][64 * k + 4 * b];
+    };
+    auto step = [&](int k, const Raw<BITS> &raw, bool live) {
+        float w[4];
+        widen<BITS, CODEBOOK>(a, raw, w);
+#pragma unroll
+        for (int q = 0; q < 4; q++) w[q] = live ? w[q] : 0.0f;
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+            f32x4 p[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                p[q] = __builtin_amdgcn_mfma_f32_4x4x1f32(xv[k & 1][g][q], w[q], f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[g][q] = acc[g][q] + p[q];
+        }
+    };
+    const int chunks = (steps + KC - 1) / KC, rest = steps - KC * (chunks - 1);  // `rest` steps in the last chunk
+    stage(0, 0);
+    load(0, cur);
+    for (int c = 0; c < chunks; c++) {
+        // Chunk c has landed for every wave, and nobody reads the buffer of
+        // chunk c - 1 any more.
+        __builtin_amdgcn_s_waitcnt(0 | 0x7 << 4 | 0xF << 8);  // vmcnt(0)
+        __syncthreads();
+        // (the weights' loads run past the end, on the last step: a load under
+        // a condition would have to be waited for at once)
+        load(c + 1, next);
+        if (c + 1 < chunks) {
+            stage(c + 1, (c + 1) & 1);
+        } else if (rest < KC) {
+            // steps past the end: columns and weights of 0, which no partial sum notices
+            for (int t = wave; t < T; t += 4)
+                for (int col = 64 * rest + lane; col < 64 * KC; col += 64) s_x[c & 1][t][col] = 0.0f;
+            __syncthreads();
+        }
+#pragma unroll
+        for (int k = 0; k < KC; k++) {
+            if (k == 0) read_x(c & 1, 0);
+            if (k + 1 < KC) read_x(c & 1, k + 1);
+            // (one step's products at a time: the accumulators leave no room for more)
+            __builtin_amdgcn_sched_barrier(0);
+            step(k, cur[k], KC * c + k < steps);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int k = 0; k < KC; k++) cur[k] = next[k];
+    }
+    const int quarter = lane >> 4, token = quarter == 1 ? 2 : quarter == 2 ? 1 : quarter;
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        const float y = tree_columns(acc[g]);
+        const int t = t0 + 4 * g + token;
+        if ((lane & 15) < 4 && r0 + i < a.rows && t < a.tokens) a.Y[(int64_t)t * a.stride + a.out + r0 + i] = y;
+    }
+}
+
+template <int BITS, bool CODEBOOK>
+void launch(sm_ctx *ctx, const ProjectArgs &a, int ng) {
+    const dim3 grid((unsigned)((a.rows + 15) / 16), (unsigned)((a.tokens + 4 * ng - 1) / (4 * ng)));
+    switch (ng) {
+        case 1: k_project_batch<BITS, CODEBOOK, 1><<<grid, 256, 0, ctx->stream>>>(a); break;
+        case 2: k_project_batch<BITS, CODEBOOK, 2><<<grid, 256, 0, ctx->stream>>>(a); break;
+        default: k_project_batch<BITS, CODEBOOK, 4><<<grid, 256, 0, ctx->stream>>>(a); break;
+    }
+}
+
+}  // namespace
+
+namespace smi {
+
+bool project_batch_takes(int bits, int cols, int tokens, uint64_t X, uint64_t codes, int group, int bias, int codebook) {
+    if (tokens < 2 || cols % 64 || X % 16 || codes % 8) return false;
+    if (bits == 16) return true;
+    if (group < 4 || (group & (group - 1)) || (codebook == 1 && bits != 4)) return false;
+    return bias > -(1 << 23) && bias < (1 << 23) - 256;
+}
+
+int project_batch(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets,
+                  float *Y, int cols, int rows, int tokens, int stride, int out, int group, int bias, int codebook,
+                  int has_offset) {
+    ProjectArgs a = {X, (const uint8_t *)codes, scales, offsets, Y, cols, rows, tokens, stride, out, 0, has_offset, (float)bias};
+    while (bits != 16 && (1 << a.group_shift) < group) a.group_shift++;
+    // Groups of tokens per wave. More of them share a weight's load and
+    // widening, fewer make more blocks. Measured at 2,560 columns, a block
+    // takes 8 / 10 / 17 us (1 / 2 / 4 groups) where every CU has one, and
+    // 5 / 5 / 7 us for each further one a CU has to take; the least of those
+    // sums is taken. bf16, in us with 1 / 2 / 4 groups: 10,240 rows x 4
+    // tokens 17 / 20 / 31, x 16 54 / 31 / 31, x 32 105 / 58 / 49; 2,560 rows
+    // x 12 12 / 14 / 17, x 16 18 / 14 / 17, x 32 28 / 20 / 23; 600 rows x 16
+    // 10.5 / 10.7 / 17.
+    const int first[3] = {8, 10, 17}, further[3] = {5, 5, 7};
+    int ng = 1, best = 0;
+    for (int k = 0; k < 3; k++) {
+        const int64_t blocks = (int64_t)((rows + 15) / 16) * ((tokens + (4 << k) - 1) / (4 << k));
+        const int cost = first[k] + further[k] * (int)std::min<int64_t>((blocks - 1) / 256, 1 << 20);
+        if (k == 0 || cost < best) {
+            ng = 1 << k;
+            best = cost;
+        }
+    }
+    switch (bits) {
+        case 2: launch<2, false>(ctx, a, ng); break;
+        case 4: codebook == 1 ? launch<4, true>(ctx, a, ng) : launch<4, false>(ctx, a, ng); break;
+        case 8: launch<8, false>(ctx, a, ng); break;
+        default: launch<16, false>(ctx, a, ng); break;
+    }
+    return launched(ctx);
+}
+
+}  // namespace smi

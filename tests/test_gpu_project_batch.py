@@ -1,0 +1,70 @@
+"""Dense projections of a token batch on the GPU against the CPU oracle, bit for
+bit: strata_bf16_project and strata_quant_project at the edges of the batch
+kernel's tiles (4 weight rows a wave and 16 a block, groups of 4 tokens up to
+32, chunks of 4 x 64 columns and what is left of them) and, at one column count
+that is no multiple of 64, of the general kernel."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # cols, rows, tokens
+    (64, 1, 2), (64, 17, 33), (128, 15, 3), (192, 16, 4), (320, 65, 5), (704, 300, 8), (640, 33, 9), (2560, 4100, 16),
+    (3072, 50, 17), (1216, 8200, 32), (100, 20, 6)]
+
+
+def same(a, b):
+    nan = np.isnan(b)
+    assert np.array_equal(np.isnan(a), nan)
+    assert np.array_equal(a.view(np.uint32)[~nan], b.view(np.uint32)[~nan])
+
+
+def inputs(cols, rows, tokens):
+    """Rows of ordinary, tiny (their products are subnormal or underflow) and huge values, and a few zeros and infinities."""
+    rng = np.random.default_rng(cols + rows + tokens)
+    x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    x[tokens // 2] *= np.float32(1e-38)
+    x[-1] *= np.float32(1e30)
+    x[0, :: max(cols // 7, 1)] = -0.0
+    if tokens > 2:
+        x[1, cols - 1] = np.inf
+    return rng, x.reshape(-1)
+
+
+@pytest.mark.parametrize("cols,rows,tokens", SHAPES)
+def test_bf16_batch(backend, oracle, cols, rows, tokens):
+    rng, x = inputs(cols, rows, tokens)
+    w = rng.normal(0, 0.05, rows * cols).astype(np.float32)
+    w[rows * cols // 2] = np.inf
+    w[rows * cols // 3] = -1e-39
+    half = (w.view(np.uint32) >> 16).astype(np.uint32)
+    codes = half[0::2] | half[1::2] << 16
+    stride, off = rows + 3, 2
+    y = backend.alloc(np.full(tokens * stride, -7, np.float32))
+    backend.run("strata_bf16_project", {"X": backend.alloc(x), "Codes": backend.alloc(codes, "u32"), "Y": y, "cols": cols,
+                                        "rows": rows, "tokens": tokens, "outputStride": stride, "outputOffset": off},
+                [rows, tokens, 1])
+    want = oracle.bf16_project(x, codes, cols, rows, tokens, stride, off, Y=np.full(tokens * stride, -7, np.float32))
+    same(backend.read(y), want)
+
+
+@pytest.mark.parametrize("cols,rows,tokens", SHAPES)
+@pytest.mark.parametrize("nbits,group,codebook,offset", [(4, 32, 0, 1), (8, 32, 0, 1), (4, 64, 1, 0), (2, 4, 0, 0),
+                                                         (8, 20, 0, 1)])
+def test_quant_batch(backend, oracle, cols, rows, tokens, nbits, group, codebook, offset):
+    if cols % group:
+        group = 4
+    rng, x = inputs(cols, rows, tokens)
+    codes = rng.integers(0, 1 << 32, (rows * cols * nbits + 31) // 32, dtype=np.uint32)
+    scales = rng.normal(0, 0.02, rows * cols // group).astype(np.float32)
+    offsets = rng.normal(0, 0.01, scales.size).astype(np.float32)
+    stride, off, bias = rows + 3, 2, -(1 << (nbits - 1))
+    y = backend.alloc(np.full(tokens * stride, -7, np.float32))
+    backend.run("strata_quant_project",
+                {"X": backend.alloc(x), "Codes": backend.alloc(codes, "u32"), "Scales": backend.alloc(scales),
+                 "Offsets": backend.alloc(offsets), "Y": y, "cols": cols, "rows": rows, "tokens": tokens,
+                 "outputStride": stride, "outputOffset": off, "bits": nbits, "groupSize": group, "bias": bias,
+                 "codebook": codebook, "hasOffset": offset}, [rows, tokens, 1])
+    want = oracle.quant_project(x, codes, scales, offsets, np.full(tokens * stride, -7, np.float32), cols, rows, tokens,
+                                stride, off, nbits, group, bias, codebook, offset)
+    same(backend.read(y), want)
