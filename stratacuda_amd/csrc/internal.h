@@ -29,7 +29,8 @@ struct sm_ctx {
     // decode layer's hand-off counters, go words and sticky fault word.
     uint32_t *counters = nullptr;
     // Scores of the batched prompt attention (strata_attention_batch):
-    // tokens x heads x 2,048 cells, kAttnScoresBytes, allocated by sm_init.
+    // tokens x heads x 2,048 cells, kAttnScoresBytes, then a float for each
+    // of those rows (their sums of exponentials); allocated by sm_init.
     float *attn_scores = nullptr;
     uint64_t launches = 0, bytes_written = 0, bytes_read = 0, allocated = 0;
     // Stage timing (sm_stage_timing): events recorded at stage boundaries.
@@ -214,8 +215,9 @@ class StaticScratchCall {
     std::lock_guard<std::mutex> lock_;
     bool capturing_ = false;
 };
-// Size of ctx->attn_scores: 1,024 (token, head) rows of 2,048 cells.
-constexpr uint64_t kAttnScoresBytes = 1024ull * 2048 * 4;
+// Scores in ctx->attn_scores: 1,024 (token, head) rows of 2,048 cells.
+constexpr uint64_t kAttnScoresRows = 1024;
+constexpr uint64_t kAttnScoresBytes = kAttnScoresRows * 2048 * 4;
 int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias, uint64_t arena,
                 uint64_t blob_stride, uint64_t shared_blob, uint64_t Wsg, int width, int ff, int experts,
                 int topk, uint64_t Y, uint64_t ids, uint64_t weights, uint64_t workspace,

@@ -528,258 +528,432 @@ __global__ __launch_bounds__(256) void k_attention_batch4(const float *__restric
     Y[(int64_t)(token * heads + h) * dim + d] = value / total;
 }
 
-// The batched prompt attention in two launches, the same operations in the
-// same order as k_attention_batch4 (kernels/strata.cu:512-534), with the
-// work spread over the GPU:
-//  k_attn_scores: one block per (64-cell tile, KV head, token). The tile's
-//    keys (64 rows) go to LDS with 16-byte loads, the query rows of the KV
-//    head's query heads too; lane l of wave w forms cell c0 + l's score for
-//    query heads w, w + 4, ... (HPW of them side by side, each the
-//    sequential dot over the head dimension), times `scale`, into
-//    S[token][head][cell].
-//  k_attn_values: below.
-// A row of keys in LDS is padded by 4 floats so that the 64 lanes' 16-byte
-// reads of one offset spread over the banks.
-template <int D, int HPW>
-__global__ __launch_bounds__(256) void k_attn_scores(const float *__restrict__ Q, const float *__restrict__ Keys,
-                                                     float *__restrict__ S, int heads, int kvHeads, int position,
-                                                     float scale, int hu) {
-    constexpr int P = D + 4;
-    __shared__ __attribute__((aligned(16))) float s_k[64 * P];
-    __shared__ __attribute__((aligned(16))) float s_q[4 * HPW][D];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int token = blockIdx.z, kh = blockIdx.y, c0 = blockIdx.x * 64, count = position + token + 1;
-    if (c0 >= count) return;
-    const int group = heads / kvHeads, h0 = kh * group;
-    for (int idx = tid; idx < 64 * (D / 4); idx += 256) {
-        const int r = idx / (D / 4), i4 = idx - r * (D / 4), cell = min(c0 + r, count - 1);
-        *(float4 *)&s_k[r * P + 4 * i4] = ((const float4 *)(Keys + ((int64_t)cell * kvHeads + kh) * D))[i4];
-    }
-    for (int idx = tid; idx < group * (D / 4); idx += 256) {
-        const int g = idx / (D / 4), i4 = idx - g * (D / 4);
-        *(float4 *)&s_q[g][4 * i4] = ((const float4 *)(Q + ((int64_t)token * heads + h0 + g) * D))[i4];
-    }
-    __syncthreads();
-    float score[HPW];
+// The batched prompt attention in three launches, the same operations in the
+// same order as k_attention_batch4 (kernels/strata.cu:512-534), spread over
+// the GPU. Every score is one sum over the head dimension and every output
+// one sum over the cells, step by step in order; only the products of a step
+// are free. v_mfma_f32_4x4x1_16b_f32 with a zero accumulator forms them
+// (each one f32 product, rounded to nearest even; a product of -0 becomes
+// +0, which a sum that starts at +0 cannot tell apart): with lane l giving
+// row l % 4's factor and column l's, register r of lane l is row r x column
+// l, so one matrix instruction serves a step of four rows' sums in 64
+// columns and the vector unit is left with the adds.
+//
+//  k_attn_scores: one block per (64-cell tile, 16 (token, head) rows of one
+//    KV head), a wave per four rows, a cell per lane; scores times `scale`
+//    into S[token][head][cell]. Bound by vector issue (22
+//    instructions for four dimensions, 3 waves a SIMD at 16 tokens x 24 heads
+//    x 2,048 cells).
+//  k_attn_softmax: one block per (token, head): S becomes the exponentials,
+//    with 0 in the rest of the last 64 cells, and their sum goes to Total.
+//  k_attn_values: a wave per RW rows of one token and 64 components. Bound by
+//    the order, 2,048 steps a sum: a matrix instruction (11 cycles), an add a
+//    row (4.5 each, a wave alone on its SIMD) and the LDS reads of a step; 20
+//    us of its 35 remain without the reads and the staging.
+// Measured at dimension 256, 24 heads on 2 KV heads, 16 tokens, 2,048 cells,
+// in us: scores 25 -> 13, softmax and values 53 -> 6 + 35 (was: vector
+// multiplies, and the softmax formed again for each of the four component
+// tiles). Not kept, values: the products on the vector unit with one row a
+// wave, exponentials from LDS (41: the reads take the LDS's whole rate) or as
+// scalars (40), stages by DMA (59).
+typedef float attn_x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ attn_x4 attn_products(float a, float b) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, attn_x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+}
+// 16 bytes per lane from global memory into LDS (lane l's at base + 16 l).
+__device__ __forceinline__ void lds_dma16(const void *src, void *lds_base) {
+    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)lds_base, 16, 0, 0);
+}
+// Every wave's LDS accesses are done, and with DMA its loads into LDS too;
+// the empty asm statements keep LDS accesses from moving across.
+template <bool DMA = false>
+__device__ __forceinline__ void attn_arrive() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x7 << 4 | (DMA ? 0 : 0xF | 3 << 14));  // lgkmcnt(0), vmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// The scores' two stages in LDS, each its own object at namespace scope: the
+// compiler then tells the loads into one from the reads of the other (with
+// one array it waits for every load before any read). Rows are 64 values in
+// sixteen 16-byte parts, part c of row r at c ^ (r % 16), so that lanes
+// reading one part of different rows meet different banks.
+struct AttnScoreStage {
+    float k[64][64], q[16][64];
+};
+__shared__ __attribute__((aligned(16))) AttnScoreStage g_attn_s0, g_attn_s1;
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void k_attn_scores(const float *__restrict__ Q, const float *__restrict__ Keys,
+                                                        float *__restrict__ S, int heads, int kvHeads, int position,
+                                                        int tokens, float scale, int hu) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c0 = blockIdx.x * 64, kh = blockIdx.y, group = heads / kvHeads, rows = tokens * group;
+    const int r0 = blockIdx.z * 16, cells = position + tokens;
+    // (the whole tile lies past its last row's cells)
+    if (c0 > position + min(r0 + 15, rows - 1) / group) return;
+    const int part = lane & 15, quarter = lane >> 4;
+    // Sources of this lane's loads: row 16 w + 4 u + quarter of the keys' tile,
+    // and row 4 w + quarter of the 16 queries (row -> token, head of KV head).
+    const float *ksrc[4];
 #pragma unroll
-    for (int u = 0; u < HPW; u++) score[u] = 0.0f;
-    const float *kr = &s_k[lane * P];
-    for (int j = 0; j < D; j += 4) {
-        const float4 k4 = *(const float4 *)&kr[j];
+    for (int u = 0; u < 4; u++) {
+        const int r = 16 * w + 4 * u + quarter;
+        ksrc[u] = Keys + ((int64_t)min(c0 + r, cells - 1) * kvHeads + kh) * D + 4 * (part ^ (r & 15));
+    }
+    const int qr = 4 * w + quarter, qrow = min(r0 + qr, rows - 1), qt = qrow / group;
+    const float *qsrc = Q + ((int64_t)qt * heads + kh * group + (qrow - qt * group)) * D + 4 * (part ^ qr);
+    auto stage = [&](AttnScoreStage &sg, int c) {
 #pragma unroll
-        for (int u = 0; u < HPW; u++) {
-            const int g = min(w + 4 * u, group - 1);
-            const float4 q4 = *(const float4 *)&s_q[g][j];
-            float v = score[u];
-            v = v + q4.x * k4.x;
-            v = v + q4.y * k4.y;
-            v = v + q4.z * k4.z;
-            v = v + q4.w * k4.w;
-            score[u] = v;
+        for (int u = 0; u < 4; u++) lds_dma16(ksrc[u] + 64 * c, &sg.k[16 * w + 4 * u][0]);
+        lds_dma16(qsrc + 64 * c, &sg.q[4 * w][0]);
+    };
+    attn_x4 score = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto sum = [&](const AttnScoreStage &sg) {
+        // a part's factors are read two steps before their products are added
+        const int r = 4 * w + (lane & 3);
+        attn_x4 k4[16], q4[16], d[2][4];
+        auto read = [&](int p) __attribute__((always_inline)) {
+            k4[p] = *(const attn_x4 *)&sg.k[lane][4 * (p ^ part)];
+            q4[p] = *(const attn_x4 *)&sg.q[r][4 * (p ^ r)];
+        };
+        auto multiply = [&](int p) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) d[p & 1][u] = attn_products(q4[p][u], k4[p][u]);
+        };
+        read(0);
+        read(1);
+        read(2);
+        multiply(0);
+#pragma unroll
+        for (int p = 0; p < 16; p++) {
+            if (p + 3 < 16) read(p + 3);
+            if (p + 1 < 16) multiply(p + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; u++) score = score + d[p & 1][u];
         }
+    };
+    stage(g_attn_s0, 0);
+#pragma unroll
+    for (int c = 0; c < D / 64; c++) {
+        attn_arrive<true>();
+        if (c + 1 < D / 64) stage(c & 1 ? g_attn_s0 : g_attn_s1, c + 1);
+        sum(c & 1 ? g_attn_s1 : g_attn_s0);
     }
     const int cell = c0 + lane;
 #pragma unroll
-    for (int u = 0; u < HPW; u++) {
-        const int g = w + 4 * u, h = h0 + g;
-        if (g < group && h < hu && cell < count) S[((int64_t)token * heads + h) * 2048 + cell] = score[u] * scale;
+    for (int u = 0; u < 4; u++) {
+        const int r = r0 + 4 * w + u, t = r / group, h = kh * group + r - t * group;
+        if (r < rows && h < hu && cell < position + t + 1) S[((int64_t)t * heads + h) * 2048 + cell] = score[u] * scale;
     }
 }
 
-// k_attn_values: one block per (64-component tile, group of up to HPW query
-// heads of one KV head, token); wave w handles head w of the group. First
-// the reference's softmax of its scores: the maximum, the exponentials and
-// their sum in the reference's lane order (lane l: cells l, l + 64, ...; the
-// tree), the probabilities in LDS. Then the weighted sum over the cells of
-// the tile's 64 components: the block's waves share the values, staged
-// through LDS 16 HPW cells at a time by all threads (double-buffered: the
-// next chunk's loads are in flight while this one is summed, and the
-// barriers order LDS only, so they do not wait for them); each lane's sum
-// runs over the cells in order.
-template <int D, int HPW>
-__global__ __launch_bounds__(64 * HPW) void k_attn_values(const float *__restrict__ S, const float *__restrict__ Values,
-                                                         float *__restrict__ Y, int heads, int kvHeads, int position,
-                                                         int hu, int tiles) {
-    constexpr int CH = 16 * HPW;  // cells per chunk: four 16-byte loads per thread
-    __shared__ __attribute__((aligned(16))) float s_p[HPW][2048];
-    __shared__ __attribute__((aligned(16))) float s_v[2][CH][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int token = blockIdx.z, count = position + token + 1, group = heads / kvHeads;
-    const int groups_per_kv = (group + HPW - 1) / HPW;
-    const int kh = blockIdx.y / groups_per_kv, g = (blockIdx.y - kh * groups_per_kv) * HPW + w;
-    const int h = kh * group + g;
-    const bool live = g < group && h < hu;
-    // (all 32 of the lane's scores loaded at once, clamped past the count)
-    const float *sc = S + ((int64_t)token * heads + min(h, heads - 1)) * 2048;
-    float sv[32];
+// The reference's softmax of one row of scores: the maximum, the exponentials
+// and their sum in the reference's lane order (lane l: cells l, l + 64, ...;
+// the tree). Wave w forms the exponentials of the 64-cell groups w, w + 4, ...
+__global__ __launch_bounds__(256) void k_attn_softmax(float *__restrict__ S, float *__restrict__ Total, int heads,
+                                                      int position) {
+    __shared__ float s_p[2048], s_mx[4];
+    __shared__ uint64_t s_tab[32];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, count = position + (int)blockIdx.y + 1;
+    const int64_t row = (int64_t)blockIdx.y * heads + blockIdx.x;
+    float *sc = S + row * 2048;
+    float v[8], mx = kNegBig;
 #pragma unroll
-    for (int i = 0; i < 32; i++) sv[i] = sc[min(lane + 64 * i, count - 1)];
-    float mx = kNegBig;
+    for (int i = 0; i < 8; i++) v[i] = sc[min(lane + 64 * (w + 4 * i), count - 1)];
+    sm::fill_exp_table(s_tab);
 #pragma unroll
-    for (int i = 0; i < 32; i++)
-        if (lane + 64 * i < count) mx = fmaxf(mx, sv[i]);
-    for (int s = 32; s > 0; s >>= 1) mx = fmaxf(mx, __shfl_down(mx, s, 64));
-    mx = __shfl(mx, 0, 64);
-    float sum = 0.0f;
+    for (int i = 0; i < 8; i++) mx = fmaxf(mx, v[i]);  // (past the count: the last score again)
+    for (int s = 32; s > 0; s >>= 1) mx = fmaxf(mx, __shfl_xor(mx, s, 64));
+    if (lane == 0) s_mx[w] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(s_mx[0], s_mx[1]), fmaxf(s_mx[2], s_mx[3]));
 #pragma unroll
-    for (int i = 0; i < 32; i++) {
-        if (lane + 64 * i < count) {
-            const float p = sm::expf_or(sv[i] - mx);
-            s_p[w][lane + 64 * i] = p;
-            sum = sum + p;
+    for (int i = 0; i < 8; i++) {
+        const int t0 = 64 * (w + 4 * i);
+        if (t0 < count) {
+            const float p = t0 + lane < count ? sm::expf_or(v[i] - mx, s_tab) : 0.0f;
+            s_p[t0 + lane] = p;
+            sc[t0 + lane] = p;
         }
     }
-    const float total = __shfl(sm::tree_sum64(sum), 0, 64);
-    const int d = blockIdx.x * 64 + lane;
-    const int64_t vstride = (int64_t)kvHeads * D;
-    const float *vtile = Values + (int64_t)kh * D + blockIdx.x * 64;
-    const int nch = (count + CH - 1) / CH;
-    // (four named registers, not an array: the compiler can place a small
-    // private array in LDS, and then waits for the loads at once)
-    const int row = threadIdx.x / 16, col = 4 * (threadIdx.x & 15);  // 16 threads per cell row
-    constexpr int RS = 4 * HPW;  // cell rows between a thread's four loads
-    auto vload = [&](int cell) -> float4 {
-        return *(const float4 *)(vtile + (int64_t)min(cell, count - 1) * vstride + col);
+    __syncthreads();
+    if (w == 0) {
+        float sum = 0.0f;
+        for (int t = lane; t < count; t += 64) sum = sum + s_p[t];
+        sum = sm::tree_sum64(sum);
+        if (lane == 0) Total[row] = sum;
+    }
+}
+
+// Grid: x = groups of four row tiles (RW heads of one token each, token by
+// token; a wave per row tile), y = component tiles, z = KV heads. (With the
+// component tiles first, each XCD met one 256-byte column of the values, which
+// lies in two of its L2's sixteen channels.) The block's waves share the
+// values, 64 cells at a time: chunk c + 1 goes from registers to the other LDS
+// buffer, and chunk c + 3's loads are issued, before chunk c is summed. (DMA
+// into LDS would save the registers, but in a loop the compiler waits for all
+// of it before the reads.) The exponentials of a wave's rows travel the same
+// way, into its own part of the buffer.
+template <int D, int RW>
+__global__ __launch_bounds__(256, 2) void k_attn_values(const float *__restrict__ S, const float *__restrict__ Total,
+                                                        const float *__restrict__ Values, float *__restrict__ Y,
+                                                        int heads, int kvHeads, int position, int tokens, int hu) {
+    __shared__ __attribute__((aligned(16))) float s_v[2][64][64], s_p[2][4][4][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kh = blockIdx.z, group = heads / kvHeads, per = (group + RW - 1) / RW, tiles = tokens * per;
+    const int last = min((int)blockIdx.x * 4 + 3, tiles - 1), tile = min((int)blockIdx.x * 4 + w, last);
+    const int token = tile / per, g0 = (tile - token * per) * RW, count = position + token + 1;
+    const int chunks = (position + last / per + 1 + 63) / 64;  // of the block's last token
+    const int64_t row0 = (int64_t)token * heads + kh * group, vstride = (int64_t)kvHeads * D;
+    const int cells = position + tokens, part = lane & 15, quarter = lane >> 4;
+    const float *vtile = Values + (int64_t)kh * D + blockIdx.y * 64 + 4 * part;
+    // (RW < 4: lanes past the wave's rows bring a row again)
+    const float *prow = S + (row0 + min(g0 + quarter % RW, group - 1)) * 2048 + 4 * part;
+    struct Chunk {
+        attn_x4 v0, v1, v2, v3, p;
     };
-    float4 l0 = vload(row), l1 = vload(row + RS), l2 = vload(row + 2 * RS), l3 = vload(row + 3 * RS);
-    *(float4 *)&s_v[0][row][col] = l0;
-    *(float4 *)&s_v[0][row + RS][col] = l1;
-    *(float4 *)&s_v[0][row + 2 * RS][col] = l2;
-    *(float4 *)&s_v[0][row + 3 * RS][col] = l3;
-    float value = 0.0f;
-    for (int c = 0; c < nch; c++) {
-        if (c + 1 < nch) {
-            const int c1 = (c + 1) * CH + row;
-            l0 = vload(c1);
-            l1 = vload(c1 + RS);
-            l2 = vload(c1 + 2 * RS);
-            l3 = vload(c1 + 3 * RS);
-        }
-        // (the next chunk's loads are issued here, not sunk to their use)
-        asm volatile("" ::: "memory");
-        sm::lds_barrier();  // chunk c is in LDS (and the probabilities); chunk c - 1's buffer is free
-        const int t0 = c * CH, n = min(CH, count - t0), buf = c & 1;
-        // 16 cells at a time: their values and probabilities read from LDS
-        // into registers, then the 16 steps of the sum
-        for (int gg = 0; gg < n; gg += 16) {
-            float vv[16], pp[16];
+    auto load = [&](int c, Chunk &l) __attribute__((always_inline)) {
+        const int cell0 = 64 * min(c, chunks - 1), r = cell0 + 16 * w + quarter;  // (past the end: the last chunk again)
+        l.v0 = *(const attn_x4 *)(vtile + min(r, cells - 1) * vstride);
+        l.v1 = *(const attn_x4 *)(vtile + min(r + 4, cells - 1) * vstride);
+        l.v2 = *(const attn_x4 *)(vtile + min(r + 8, cells - 1) * vstride);
+        l.v3 = *(const attn_x4 *)(vtile + min(r + 12, cells - 1) * vstride);
+        l.p = *(const attn_x4 *)(prow + cell0);
+    };
+    auto store = [&](int buf, const Chunk &l) __attribute__((always_inline)) {
+        float *at = &s_v[buf][16 * w + quarter][4 * part];
+        *(attn_x4 *)at = l.v0;
+        *(attn_x4 *)(at + 4 * 64) = l.v1;
+        *(attn_x4 *)(at + 8 * 64) = l.v2;
+        *(attn_x4 *)(at + 12 * 64) = l.v3;
+        *(attn_x4 *)&s_p[buf][w][quarter][4 * (part ^ quarter)] = l.p;  // (rows on different banks)
+    };
+    attn_x4 value = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int qr = lane & 3;
+    // Four cells at a time: their factors are read three steps before their
+    // products are added, the products formed one step before.
+    struct Four {
+        attn_x4 p, v;
+    };
+    auto read4 = [&](int buf, int i) __attribute__((always_inline)) {
+        Four f;
+        f.p = *(const attn_x4 *)&s_p[buf][w][qr][4 * (i ^ qr)];
 #pragma unroll
-            for (int u = 0; u < 16; u++) vv[u] = s_v[buf][min(gg + u, CH - 1)][lane];
+        for (int u = 0; u < 4; u++) f.v[u] = s_v[buf][4 * i + u][lane];
+        return f;
+    };
+    auto multiply4 = [&](const Four &f, attn_x4(&d)[4]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 p4 = *(const float4 *)&s_p[w][min(t0 + gg + 4 * i, 2044)];
-                pp[4 * i] = p4.x;
-                pp[4 * i + 1] = p4.y;
-                pp[4 * i + 2] = p4.z;
-                pp[4 * i + 3] = p4.w;
+        for (int u = 0; u < 4; u++) d[u] = attn_products(f.p[u], f.v[u]);
+    };
+    auto add4 = [&](const attn_x4(&d)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int r = 0; r < RW; r++) value[r] = value[r] + d[u][r];
+        // (all four registers of a product stay its own until here: with the
+        // unused ones shared, the next product would have to wait for this one)
+#pragma unroll
+        for (int u = 0; u < 4; u++) asm volatile("" : : "v"(d[u]));
+    };
+    auto chunk = [&](int c, int buf, Chunk &l) __attribute__((always_inline)) {
+        attn_arrive();
+        const int left = count - 64 * c;
+        Four f[16];
+        attn_x4 d[2][4];
+        f[0] = read4(buf, 0);
+        f[1] = read4(buf, 1);
+        f[2] = read4(buf, 2);
+        store(buf ^ 1, l);
+        load(c + 3, l);
+        if (left >= 64) {
+            multiply4(f[0], d[0]);
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                if (i + 3 < 16) f[i + 3] = read4(buf, i + 3);
+                if (i + 1 < 16) multiply4(f[i + 1], d[(i + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                add4(d[i & 1]);
             }
-            if (gg + 16 <= n) {
+        } else {
+#pragma clang loop unroll(disable)
+            for (int i = 0; 4 * i < left; i++) {
+                Four g = read4(buf, i);
+                // (cells past the count: 0 x 0, which no sum notices)
 #pragma unroll
-                for (int u = 0; u < 16; u++) value = value + pp[u] * vv[u];
-            } else {
-                for (int u = 0; u < n - gg; u++) {
-                    float a = pp[0], b = vv[0];
-#pragma unroll
-                    for (int i = 1; i < 16; i++) {
-                        a = u == i ? pp[i] : a;
-                        b = u == i ? vv[i] : b;
-                    }
-                    value = value + a * b;
-                }
+                for (int u = 1; u < 4; u++) g.v[u] = 4 * i + u < left ? g.v[u] : 0.0f;
+                multiply4(g, d[0]);
+                add4(d[0]);
             }
         }
-        // the next chunk goes to LDS only after this one is summed (its loads
-        // were in flight meanwhile)
-        asm volatile("" ::: "memory");
-        if (c + 1 < nch) {
-            const int nb = (c + 1) & 1;
-            *(float4 *)&s_v[nb][row][col] = l0;
-            *(float4 *)&s_v[nb][row + RS][col] = l1;
-            *(float4 *)&s_v[nb][row + 2 * RS][col] = l2;
-            *(float4 *)&s_v[nb][row + 3 * RS][col] = l3;
-        }
+    };
+    Chunk even, odd;  // chunks still in registers
+    load(0, even);
+    load(1, odd);
+    store(0, even);
+    load(2, even);
+    for (int c = 0;; c += 2) {
+        chunk(c, 0, odd);
+        if (c + 1 >= chunks) break;
+        chunk(c + 1, 1, even);
+        if (c + 2 >= chunks) break;
     }
-    if (live && blockIdx.x < (unsigned)tiles && d < D) Y[((int64_t)token * heads + h) * D + d] = value / total;
+    const int d = blockIdx.y * 64 + lane;
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+        const int g = g0 + r, h = kh * group + g;
+        if ((int)blockIdx.x * 4 + w <= last && g < group && h < hu) Y[(row0 + g) * D + d] = value[r] / Total[row0 + g];
+    }
 }
 
-// k_gdn_batch_reg with the key and query rows of the block's key head staged
-// in LDS (16 tokens at a time) and one 64-thread block per 64 state columns
-// (all of one value head: D is a multiple of 64), so that each of the
-// column's two sequential sums per token reads its K / Q values from LDS
-// instead of waiting on global loads, and the columns spread over the CUs.
-// The K / Q rows arrive by DMA, Decay and Beta of the staged tokens with
-// them, and each token's V value one token ahead. The same operations in the
-// same order as the reference (kernels/strata.cu:432-445). At the
-// production shape (6,144 columns: 96 waves) each wave runs two dependent
-// 128-step sums per token; the kernel is bound by that latency.
+// k_gdn_batch_reg for whole value heads (D = 64 or 128), with a state column
+// spread over eight lanes: lane 8 c + p of a wave holds values R p .. R p +
+// R - 1 (R = D / 8) of the wave's column c. The same operations in the same
+// order as the reference (kernels/strata.cu:432-445); what bounds it is the
+// order, two sums of D dependent steps per token. Products, decays and
+// updates are R per lane instead of D. A sum passes through the eight lanes:
+// all lanes add their own R products to what their left neighbour holds,
+// eight times over, and after round p lane p is right, so the last lane ends
+// with the sum (D adds, the hand-over a DPP operand of the first of a
+// round). A token's result and the next token's prediction both follow from
+// the same update, so their two sums run side by side.
+//
+// The key and query rows of the block's key head arrive by DMA, 16 tokens at
+// a time, with their Decay and Beta. Measured at 6,144 columns, 16 tokens: 39
+// us with a column per lane (96 waves, 14,000 instructions each) -> 17 us (768
+// waves, 5,400 each).
 constexpr int kGdnStage = 16;
-// 16 bytes per lane from global memory into LDS (lane l's at base + 16 l).
-__device__ __forceinline__ void gdn_dma16(const void *src, void *lds_base) {
-    __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void *)lds_base, 16, 0, 0);
+constexpr int kGdnParts = 8;
+// Lane 7 of each group of eight lanes, in all eight.
+__device__ __forceinline__ float gdn_last_part(float v) {
+    const float quad = sm::dpp_f32<0xff>(v, v), other = sm::dpp_f32<sm::kDppRowHalfMirror>(quad, quad);
+    return (threadIdx.x & 4) ? quad : other;
+}
+template <int R>
+__device__ __forceinline__ void gdn_load(const float *row, float (&out)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; i += 4) {
+        const float4 v = *(const float4 *)(row + i);
+        out[i] = v.x;
+        out[i + 1] = v.y;
+        out[i + 2] = v.z;
+        out[i + 3] = v.w;
+    }
 }
 template <int D>
-__global__ void __launch_bounds__(64) k_gdn_batch_lds(float *__restrict__ State, const float *__restrict__ Q,
+__global__ void __launch_bounds__(256) k_gdn_batch_lds(float *__restrict__ State, const float *__restrict__ Q,
                                                       const float *__restrict__ K, const float *__restrict__ V,
                                                       const float *__restrict__ Decay, const float *__restrict__ Beta,
                                                       float *__restrict__ Y, int keyHeads, int valueHeads, int tokens,
                                                       int n) {
-    static_assert(D % 64 == 0 && D <= GDN_REG_MAX_DIM, "whole value heads per block group");
+    static_assert(D % 64 == 0 && D <= GDN_REG_MAX_DIM && kGdnParts == 8, "whole value heads per block group");
+    constexpr int R = D / kGdnParts, C = 256 / kGdnParts;  // values per lane, columns per block (of one value head)
     __shared__ __attribute__((aligned(16))) float s_k[kGdnStage][D], s_q[kGdnStage][D];
-    __shared__ float s_decay[kGdnStage], s_beta[kGdnStage];
-    const int jh = blockIdx.x * 64 + threadIdx.x;
-    const int h = (int)(blockIdx.x * 64) / D, kh = h % keyHeads, stride = valueHeads * D;
+    __shared__ float s_decay[kGdnStage], s_beta[kGdnStage], s_v[kGdnStage][C];
+    const int part = threadIdx.x % kGdnParts, jh = blockIdx.x * C + threadIdx.x / kGdnParts;
+    const int h = (int)(blockIdx.x * C) / D, kh = h % keyHeads, stride = valueHeads * D;
     const bool live = jh < n;
-    const int col = min(jh, n - 1);
-    float st[D];
+    const int col = min(jh, n - 1), lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float st[R];
 #pragma unroll
-    for (int i = 0; i < D; ++i) st[i] = State[(int64_t)i * stride + col];
+    for (int i = 0; i < R; ++i) st[i] = State[(int64_t)(R * part + i) * stride + col];
     for (int t0 = 0; t0 < tokens; t0 += kGdnStage) {
         const int nt = min(kGdnStage, tokens - t0);
         __syncthreads();  // the previous stage's readers are done
         // K and Q rows of the stage's tokens by DMA into LDS (16 bytes per
         // lane, a kilobyte per instruction: 1,024 / (4 D) rows; rows past
-        // the stage's tokens reload its last token and are never read)
+        // the stage's tokens reload its last token and are never used)
         constexpr int RPI = 256 / D;  // rows per instruction
-        const int lr = threadIdx.x / (D / 4), lo = 4 * (threadIdx.x % (D / 4));
+        const int lr = lane / (D / 4), lo = 4 * (lane % (D / 4));
 #pragma unroll
-        for (int i = 0; i < kGdnStage / RPI; i++) {
-            const int tt = min(RPI * i + lr, nt - 1);
+        for (int i = 0; i < kGdnStage / RPI / 4; i++) {
+            const int r0 = RPI * (4 * i + wave), tt = min(r0 + lr, nt - 1);
             const int64_t qbase = ((int64_t)(t0 + tt) * keyHeads + kh) * D + lo;
-            gdn_dma16(K + qbase, &s_k[RPI * i][0]);
-            gdn_dma16(Q + qbase, &s_q[RPI * i][0]);
+            lds_dma16(K + qbase, &s_k[r0][0]);
+            lds_dma16(Q + qbase, &s_q[r0][0]);
         }
         if (threadIdx.x < nt) {
             s_decay[threadIdx.x] = Decay[(t0 + threadIdx.x) * valueHeads + h];
             s_beta[threadIdx.x] = Beta[(t0 + threadIdx.x) * valueHeads + h];
         }
+        // (V too: a load in the token loop would have to wait for the token's store)
+#pragma unroll
+        for (int i = 0; i < kGdnStage * C / 256; i++) {
+            const int tt = 256 / C * i + threadIdx.x / C, c = threadIdx.x % C;
+            s_v[tt][c] = V[(int64_t)(t0 + min(tt, nt - 1)) * stride + min((int)blockIdx.x * C + c, n - 1)];
+        }
         __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4) | (0xf << 8));  // vmcnt(0): the DMA is in LDS
         __syncthreads();
-        // the token's V value, loaded one token ahead (one register, not a
-        // register per staged token)
-        float vnext = V[(int64_t)t0 * stride + col];
-        for (int tt = 0; tt < nt; tt++) {
-            const float vt = vnext;
-            vnext = V[(int64_t)(t0 + min(tt + 1, nt - 1)) * stride + col];
-            const float decay = s_decay[tt];
-            float prediction = 0.0f;
+        // Token tt's keys are in k[tt % 2], its queries in q, its value and
+        // strength in v and beta, and token tt + 1's decay in decay.
+        float k[2][R], q[R], a[R], b[R];
+        auto at = [&](int tt) { return min(tt, nt - 1); };
+        gdn_load<R>(&s_k[0][R * part], k[0]);
+        gdn_load<R>(&s_k[at(1)][R * part], k[1]);
+        gdn_load<R>(&s_q[0][R * part], q);
+        float decay = s_decay[0], v = s_v[0][threadIdx.x / kGdnParts], beta = s_beta[0];
+        // the stage's first prediction, alone
+        float prediction = 0.0f;
 #pragma unroll
-            for (int i = 0; i < D; ++i) {
-                st[i] = st[i] * decay;
-                prediction = prediction + st[i] * s_k[tt][i];
+        for (int i = 0; i < R; ++i) {
+            st[i] = st[i] * decay;
+            b[i] = st[i] * k[0][i];
+        }
+        decay = s_decay[at(1)];
+#pragma unroll
+        for (int p = 0; p < kGdnParts; p++) {
+            if (p > 0) prediction = sm::dpp_f32<0x111>(0.0f, prediction);  // row_shr:1
+#pragma unroll
+            for (int i = 0; i < R; ++i) prediction = prediction + b[i];
+        }
+        auto token = [&](int tt, float(&k0)[R], const float(&k1)[R]) __attribute__((always_inline)) {
+            const float delta = gdn_last_part((v - prediction) * beta);
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                st[i] = st[i] + k0[i] * delta;
+                a[i] = st[i] * q[i];
             }
-            const float delta = (vt - prediction) * s_beta[tt];
+            const bool last = tt + 1 == nt;
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const float d = st[i] * decay;
+                b[i] = d * k1[i];  // (formed for nothing after the stage's last token)
+                st[i] = last ? st[i] : d;
+            }
+            // what the next token needs is read while the sums run
+            gdn_load<R>(&s_k[at(tt + 2)][R * part], k0);
+            gdn_load<R>(&s_q[at(tt + 1)][R * part], q);
+            decay = s_decay[at(tt + 2)];
+            v = s_v[at(tt + 1)][threadIdx.x / kGdnParts];
+            beta = s_beta[at(tt + 1)];
+            __builtin_amdgcn_sched_barrier(0);
             float result = 0.0f;
+            prediction = 0.0f;
 #pragma unroll
-            for (int i = 0; i < D; ++i) {
-                st[i] = st[i] + s_k[tt][i] * delta;
-                result = result + st[i] * s_q[tt][i];
+            for (int p = 0; p < kGdnParts; p++) {
+                if (p > 0) {
+                    result = sm::dpp_f32<0x111>(0.0f, result);
+                    prediction = sm::dpp_f32<0x111>(0.0f, prediction);
+                }
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    result = result + a[i];
+                    prediction = prediction + b[i];
+                }
             }
-            if (live) Y[(int64_t)(t0 + tt) * stride + jh] = result;
+            if (live && part == kGdnParts - 1) Y[(int64_t)(t0 + tt) * stride + jh] = result;
+        };
+        for (int tt = 0; tt < nt; tt += 2) {
+            token(tt, k[0], k[1]);
+            if (tt + 1 < nt) token(tt + 1, k[1], k[0]);
         }
     }
     if (live) {
 #pragma unroll
-        for (int i = 0; i < D; ++i) State[(int64_t)i * stride + jh] = st[i];
+        for (int i = 0; i < R; ++i) State[(int64_t)(R * part + i) * stride + jh] = st[i];
     }
 }
 
@@ -1162,8 +1336,8 @@ int L_gdn_batch(sm_ctx *ctx, const uint32_t *G, Args a) {
     bool distinct = true;
     for (int i = 1; i < 7; i++) distinct = distinct && a.ptr(i) != a.ptr(0);
     if (distinct && (dim == 64 || dim == 128)) {
-        // whole value heads of 64-column blocks, K / Q staged in LDS
-        (dim == 64 ? k_gdn_batch_lds<64> : k_gdn_batch_lds<128>)<<<(unsigned)((n + 63) / 64), 64, 0, ctx->stream>>>(
+        // eight lanes a column, 32 columns (of one value head) a block
+        (dim == 64 ? k_gdn_batch_lds<64> : k_gdn_batch_lds<128>)<<<(unsigned)((n + 31) / 32), 256, 0, ctx->stream>>>(
             Fw(a, 0), F(a, 1), F(a, 2), F(a, 3), F(a, 4), F(a, 5), Fw(a, 6), keyHeads, valueHeads, tokens, (int)n);
         return launched(ctx);
     }
@@ -1242,29 +1416,30 @@ int L_attention_batch(sm_ctx *ctx, const uint32_t *G, Args a) {
     if (int rc = need(ctx, a.ptr(1), kv, "Keys")) return rc;
     if (int rc = need(ctx, a.ptr(2), kv, "Values")) return rc;
     if (int rc = need(ctx, a.ptr(3), (uint64_t)((int64_t)(tu - 1) * heads + hu) * dim * 4, "Y")) return rc;
-    // Two launches over the whole GPU (k_attn_scores, k_attn_values) for the
-    // production head sizes; one otherwise.
+    // Three launches over the whole GPU for the production head sizes; one otherwise.
     const int group = heads / kvHeads;
-    if ((dim == 64 || dim == 128 || dim == 256) && group <= 16 && (uint64_t)tu * heads * 2048 * 4 <= kAttnScoresBytes) {
-        using KS = void (*)(const float *, const float *, float *, int, int, int, float, int);
-        const int di = dim == 64 ? 0 : dim == 128 ? 1 : 2, hpw = (group + 3) / 4;
-        static const KS ks[3][4] = {{k_attn_scores<64, 1>, k_attn_scores<64, 2>, k_attn_scores<64, 3>, k_attn_scores<64, 4>},
-                                    {k_attn_scores<128, 1>, k_attn_scores<128, 2>, k_attn_scores<128, 3>,
-                                     k_attn_scores<128, 4>},
-                                    {k_attn_scores<256, 1>, k_attn_scores<256, 2>, k_attn_scores<256, 3>,
-                                     k_attn_scores<256, 4>}};
-        using KV = void (*)(const float *, const float *, float *, int, int, int, int, int);
-        const int vh = group >= 4 ? 4 : group >= 2 ? 2 : 1, vi = vh == 4 ? 2 : vh == 2 ? 1 : 0;
-        static const KV kv[3][3] = {{k_attn_values<64, 1>, k_attn_values<64, 2>, k_attn_values<64, 4>},
-                                    {k_attn_values<128, 1>, k_attn_values<128, 2>, k_attn_values<128, 4>},
-                                    {k_attn_values<256, 1>, k_attn_values<256, 2>, k_attn_values<256, 4>}};
+    if ((dim == 64 || dim == 128 || dim == 256) && (uint64_t)tu * heads * 2048 * 4 <= kAttnScoresBytes) {
+        float *totals = ctx->attn_scores + kAttnScoresBytes / 4;
+        const int di = dim == 64 ? 0 : dim == 128 ? 1 : 2;
         const int kvu = std::min(kvHeads, (hu - 1) / group + 1), cells = position + tu;
-        ks[di][hpw - 1]<<<dim3((cells + 63) / 64, kvu, tu), 256, 0, ctx->stream>>>(F(a, 0), F(a, 1), ctx->attn_scores,
-                                                                                    heads, kvHeads, position, scale, hu);
+        using KS = void (*)(const float *, const float *, float *, int, int, int, int, float, int);
+        static const KS ks[3] = {k_attn_scores<64>, k_attn_scores<128>, k_attn_scores<256>};
+        ks[di]<<<dim3((cells + 63) / 64, kvu, (tu * group + 15) / 16), 256, 0, ctx->stream>>>(
+            F(a, 0), F(a, 1), ctx->attn_scores, heads, kvHeads, position, tu, scale, hu);
         if (int rc = launched(ctx)) return rc;
-        const int gpk = (group + vh - 1) / vh;
-        kv[di][vi]<<<dim3(tiles, kvu * gpk, tu), 64 * vh, 0, ctx->stream>>>(ctx->attn_scores, F(a, 2), Fw(a, 3), heads,
-                                                                            kvHeads, position, hu, tiles);
+        k_attn_softmax<<<dim3(hu, tu), 256, 0, ctx->stream>>>(ctx->attn_scores, totals, heads, position);
+        if (int rc = launched(ctx)) return rc;
+        // Heads per wave: one while every wave has one of the 1,024 SIMDs to
+        // itself, then two (at 16 tokens, 1,536 waves of one or 768 of two:
+        // 47 or 35 us).
+        const int ri = (int64_t)tu * hu * tiles <= 1024 ? 0 : 1, rw = 1 << ri;
+        using KV = void (*)(const float *, const float *, const float *, float *, int, int, int, int, int);
+        static const KV kv[3][2] = {{k_attn_values<64, 1>, k_attn_values<64, 2>},
+                                    {k_attn_values<128, 1>, k_attn_values<128, 2>},
+                                    {k_attn_values<256, 1>, k_attn_values<256, 2>}};
+        const int row_tiles = tu * ((group + rw - 1) / rw);
+        kv[di][ri]<<<dim3((row_tiles + 3) / 4, tiles, kvu), 256, 0, ctx->stream>>>(
+            ctx->attn_scores, totals, F(a, 2), Fw(a, 3), heads, kvHeads, position, tu, hu);
         return launched(ctx);
     }
     k_attention_batch4<<<dim3(hu, (tiles + 3) / 4, tu), 256, 0, ctx->stream>>>(F(a, 0), F(a, 1), F(a, 2), Fw(a, 3),

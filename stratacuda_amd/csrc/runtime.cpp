@@ -144,7 +144,7 @@ int sm_init(int device, sm_ctx **out) {
         }
     }
     if (hipMalloc((void **)&ctx->counters, kCounterWords * sizeof(uint32_t)) != hipSuccess ||
-        hipMalloc((void **)&ctx->attn_scores, kAttnScoresBytes) != hipSuccess ||
+        hipMalloc((void **)&ctx->attn_scores, kAttnScoresBytes + kAttnScoresRows * 4) != hipSuccess ||
         hipMemset(ctx->counters, 0, kCounterWords * sizeof(uint32_t)) != hipSuccess ||
         hipDeviceSynchronize() != hipSuccess) {
         sm_shutdown(ctx);
