@@ -440,10 +440,10 @@ def _gemm_label(name):
             "gate_up" if m.group(1) == "1" else "down", 32 * int(m.group(2)), 128 * int(m.group(3)), m.group(4))
     # 16-row kernels: weight rows per block 64 x NT (the rows16 kernel's third
     # template argument, 4 when absent), mangled or demangled
-    m = re.search(r"k_moe_gemm_(stream16|rows16)ILb(\d)ELi(\d+)E(?:Li(\d)E)?", name)
+    m = re.search(r"k_moe_gemm_(rows16)ILb(\d)ELi(\d+)E(?:Li(\d)E)?", name)
     g = (m.group(1), m.group(2) == "1", m.group(3), m.group(4)) if m else None
     if not m:
-        m = re.search(r"k_moe_gemm_(stream16|rows16)<(true|false), (\d+)(?:, (\d))?>", name)
+        m = re.search(r"k_moe_gemm_(rows16)<(true|false), (\d+)(?:, (\d))?>", name)
         g = (m.group(1), m.group(2) == "true", m.group(3), m.group(4)) if m else None
     if g:
         return "k_moe_gemm_%s<%s, 16 x %d tile, K/64 = %s>" % (g[0], "gate_up" if g[1] else "down",

@@ -27,9 +27,9 @@
 //    (p, p+8) of word w come out of the code unpacking, so B needs no
 //    shuffle; the activations are stored in the same order, so staging them
 //    into LDS is a plain 16-byte copy and the MFMA A operand one 16-byte read.
-//  * Tiles (width and ff among 512 / 2048, the benchmark shapes): below 1,024
-//    tokens every segment runs in 16 x 256 blocks on v_mfma_f32_16x16x32_f16
-//    (k_moe_gemm_rows16, k_moe_gemm_stream16), one grid; from 1,024 tokens
+//  * Tiles (width a multiple of 256 up to 2,560, ff of 128; stream_groups): below
+//    1,024 tokens every segment runs in 16 x 256 blocks on
+//    v_mfma_f32_16x16x32_f16 (k_moe_gemm_rows16), one grid; from 1,024 tokens
 //    segments of more than 32 rows run in 64 x 256 blocks on
 //    v_mfma_f32_32x32x16_f16 (k_moe_gemm_stream), the two grids covering
 //    disjoint rows and running on two streams. Each block reads
@@ -43,6 +43,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <utility>
 
 #include "internal.h"
 #include "strata_device.h"
@@ -377,6 +378,13 @@ __device__ __forceinline__ void xcd_tile(int &tau, int &cb) {
 }
 
 constexpr int STREAM_MAX_G = 40;  // K <= 2560 for the streaming kernels (the real model's width)
+// K / 64 of the compiled streaming kernels: whole supersteps of the 16-row
+// kernel up to the real model's width, and even counts up to 16 in the down
+// product, whose K is an expert's hidden width (512 and 640 in the benchmark's
+// and the real model's).
+constexpr bool stream_groups(bool gate_up, int g) {
+    return g >= 2 && g <= STREAM_MAX_G && (g % 4 == 0 || (!gate_up && g % 2 == 0 && g <= 16));
+}
 
 // The G fp16 scales of one weight row (2G contiguous bytes) into G/2 words:
 // 16-byte loads when a row is a whole number of them (G % 8 == 0), else
@@ -424,28 +432,14 @@ struct Ring<64> {
         return S == 0 ? g_big0 : S == 1 ? g_big1 : g_big2;
     }
 };
-// 16-row tiles (k_moe_gemm_stream16): 8 KiB stages, six of them (48 KiB,
-// three blocks per CU).
-__shared__ __attribute__((aligned(16))) RingStage<16> g_tiny0, g_tiny1, g_tiny2, g_tiny3, g_tiny4, g_tiny5;
-template <>
-struct Ring<16> {
-    static constexpr int NS = 6;
-    template <int S>
-    static __device__ __forceinline__ RingStage<16> &stage() {
-        return S == 0 ? g_tiny0 : S == 1 ? g_tiny1 : S == 2 ? g_tiny2 : S == 3 ? g_tiny3 : S == 4 ? g_tiny4 : g_tiny5;
-    }
-};
 // Calls f(stage S) for the S equal to `slot` (slot is a constant once the
 // group loop is unrolled).
 template <int BM, typename F>
 __device__ __forceinline__ void with_stage(int slot, F &&f) {
     switch (slot) {
     case 0: f(Ring<BM>::template stage<0>()); break;
-    case 1: f(Ring<BM>::template stage<1 % Ring<BM>::NS>()); break;
-    case 2: f(Ring<BM>::template stage<2 % Ring<BM>::NS>()); break;
-    case 3: f(Ring<BM>::template stage<3 % Ring<BM>::NS>()); break;
-    case 4: f(Ring<BM>::template stage<4 % Ring<BM>::NS>()); break;
-    default: f(Ring<BM>::template stage<5 % Ring<BM>::NS>()); break;
+    case 1: f(Ring<BM>::template stage<1>()); break;
+    default: f(Ring<BM>::template stage<2>()); break;
     }
 }
 
@@ -468,7 +462,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm_stream(const _Float16 *__restr
     constexpr int BM = P::BM, BN = P::BN, ACH = P::ACH, BCH = P::BCH;
     using Stage = RingStage<BM>;
     constexpr int NS = Ring<BM>::NS;
-    static_assert(KG >= 8 && KG <= STREAM_MAX_G && KG % 2 == 0, "K / 64 groups");
+    static_assert(KG >= 2 && KG <= STREAM_MAX_G && KG % 2 == 0, "K / 64 groups");
     static_assert(BM <= 64 && BN <= 256, "stage size");
     // Tile record (segment, first row, end of the segment) from the dispatch.
     int tau, cb;
@@ -603,139 +597,14 @@ __global__ void __launch_bounds__(256) k_moe_gemm_stream(const _Float16 *__restr
             }
 }
 
-// The streaming kernel for short segments: 16-row tiles on
-// v_mfma_f32_16x16x32_f16, so a segment of ~10 rows (the typical expert at a
-// few hundred tokens) pays for 16 rows of MFMA work instead of 32. Block:
-// 16 rows x 256 weight rows, 4 waves side by side in N, each 16 x 64 (four
-// 16 x 16 tiles). The 16x16x32 operands: lane l holds row (or column) l % 16
-// and K positions 8 (l / 16) .. +7 of a 32-wide step. With the K order of the
-// activations, step s of a 64-wide group and lane quarter kq = l / 16 map to
-// code word 2s + kq / 2, byte half kq % 2 (the same unpacking as the 32-row
-// kernel's lane halves) and to the 16-byte part 4s + kq of the A row.
-// Result: lane l holds rows 4 (l / 16) + i (i = 0..3) of column l % 16.
 typedef float float4v __attribute__((ext_vector_type(4)));
-template <bool GATE_UP, int KG>
-__global__ void __launch_bounds__(256) k_moe_gemm_stream16(const _Float16 *__restrict__ A, const int *__restrict__ rows,
-                                                           const int4 *__restrict__ info,
-                                                           const int *__restrict__ tiles,
-                                                           const uint8_t *__restrict__ arena, uint64_t stride,
-                                                           const uint8_t *__restrict__ shared_blob, int experts,
-                                                           uint64_t codes_off, uint64_t scales_off, int K, int N,
-                                                           void *__restrict__ out, int out_ld) {
-    constexpr int BM = 16, BN = 256, NT = 4;  // NT tiles of 16 columns per wave
-    using Stage = RingStage<BM>;
-    constexpr int NS = Ring<BM>::NS;
-    constexpr int G = KG;  // K / 64
-    static_assert(KG >= 8 && KG <= STREAM_MAX_G && KG % 2 == 0, "K / 64 groups");
-    (void)K;
-    (void)N;
-    // Tile record (segment, first row, end of the segment) from the dispatch.
-    int tau, cb;
-    xcd_tile(tau, cb);
-    if (tau >= tiles[experts + 1]) return;
-    const int4 ti = info[tau];
-    const int e = ti.x, m0 = ti.y, mend = ti.z;
-    const uint8_t *blob = e < experts ? arena + (uint64_t)e * stride : shared_blob;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = cb * BN;
 
-    // DMA sources, one A and one B load per thread per stage. A chunk
-    // c = tid: hi/lo c / 128, row (c / 8) % 16, slot c % 8 holding part
-    // slot ^ ((row / 2) & 7).
-    const _Float16 *asrc;
-    {
-        const int hl = tid >> 7, r = (tid >> 3) & 15, part = (tid & 7) ^ ((r >> 1) & 7);
-        const int pos = min(m0 + r, mend - 1);  // rows past the end load the segment's last row
-        const int64_t arow = GATE_UP ? (e < experts ? rows[pos] : pos - ti.w) : pos;
-        asrc = A + (arow * G * 2 + hl) * 64 + part * 8;
-    }
-    const uint8_t *bsrc = blob + codes_off + (uint64_t)(n0 + tid) * (G * 16);
-    auto issue = [&](Stage &sg, int g) {
-        dma16(asrc + (int64_t)g * 128, &sg.a[64 * wave]);
-        dma16(bsrc + (uint64_t)g * 16, &sg.b[64 * wave]);
-    };
-    const int col = lane & 15, kq = lane >> 4;
-    // Scales of the lane's four weight rows, every group, in registers.
-    uint32_t sreg[NT][G / 2];
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++)
-        load_row_scales<G>(blob + scales_off + (uint64_t)(n0 + wave * 64 + nt * 16 + col) * G * 2, sreg[nt]);
-#pragma clang loop unroll(full)
-    for (int q = 0; q < NS - 1; q++) with_stage<BM>(q, [&](Stage &sg) { issue(sg, min(q, G - 1)); });
-
-    const PairMagic magic = pair_magic();
-    // Byte selector of the lane's code word: word x (kq < 2) or y, moved
-    // down by one byte for odd kq (v_perm_b32: 0-3 pick bytes of the second
-    // source, 4-7 of the first, 0x0c gives zero).
-    const uint32_t psel = kq == 0 ? 0x03020100u : kq == 1 ? 0x0c030201u : kq == 2 ? 0x07060504u : 0x0c070605u;
-    float4v acc[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) acc[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
-
-    auto compute = [&](const Stage &sg, int g) {
-        uint32_t words[NT][2];  // the lane's code word of step 0 and 1, shifted
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            const v4u cv = sg.b[wave * 64 + nt * 16 + col];
-            words[nt][0] = __builtin_amdgcn_perm(cv.y, cv.x, psel);
-            words[nt][1] = __builtin_amdgcn_perm(cv.w, cv.z, psel);
-        }
-        half2v scale[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            const uint16_t s16 = (uint16_t)(sreg[nt][g >> 1] >> (16 * (g & 1)));
-            const _Float16 sh = __builtin_bit_cast(_Float16, s16);
-            scale[nt] = (half2v){sh, sh};
-        }
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const int part = 4 * s + kq, slot = part ^ ((col >> 1) & 7);
-            const half8 ahi = __builtin_bit_cast(half8, sg.a[col * 8 + slot]);
-            const half8 alo = __builtin_bit_cast(half8, sg.a[(BM + col) * 8 + slot]);
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const half8 b = b_operand_word(words[nt][s], magic, scale[nt]);
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, b, acc[nt], 0, 0, 0);
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, b, acc[nt], 0, 0, 0);
-            }
-        }
-    };
-    constexpr int PS = 2;  // loads per thread per stage
-#pragma clang loop unroll(full)
-    for (int g = 0; g < G; g++) {
-        ring_sync<PS * (NS - 2)>();
-        with_stage<BM>((g + NS - 1) % NS, [&](Stage &sg) { issue(sg, min(g + NS - 1, G - 1)); });
-        with_stage<BM>(g % NS, [&](Stage &sg) { compute(sg, g); });
-    }
-    // No load may still be writing LDS when the block ends.
-    ring_sync<0>();
-
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int pos = m0 + 4 * kq + i, n = n0 + wave * 64 + nt * 16 + col;
-            if (GATE_UP) {
-                const float other = sm::dpp_f32<sm::kDppQuadXor1>(acc[nt][i], acc[nt][i]);
-                if ((col & 1) == 0 && pos < mend) {
-                    const float h = silu_fast(acc[nt][i]) * other;
-                    const int jj = n >> 1;
-                    _Float16 *dst =
-                        (_Float16 *)out + ((int64_t)pos * (out_ld / 64) + (jj >> 6)) * 128 + k_position(jj & 63);
-                    const _Float16 hi = (_Float16)h;
-                    dst[0] = hi;
-                    dst[64] = (_Float16)(h - (float)hi);
-                }
-            } else if (pos < mend) {
-                ((float *)out)[(int64_t)pos * out_ld + n] = acc[nt][i];
-            }
-        }
-}
-
-// The 16-row kernel for K a multiple of 256, in supersteps of four scale
-// groups. Weight codes go from HBM straight to the lanes that use them: in
-// superstep S, lane (col, kq) of wave w loads the 16 code bytes of group
-// 4S + kq of weight rows n0 + 64w + 16nt + col (nt = 0..3). One load
+// The 16-row kernel, in supersteps of four scale groups (the last of two when
+// K / 64 is not a multiple of four: the real model's down product, K = 640,
+// took 131 us at 333 tokens with a ring of single groups, 78 us so). Weight
+// codes go from HBM straight to the lanes that use them: in superstep S, lane
+// (col, kq) of wave w loads the 16 code bytes of group 4S + kq of weight rows
+// n0 + 64w + 16nt + col (nt = 0..3). One load
 // instruction then reads 64 contiguous bytes of each of 16 rows (reading 16
 // bytes of each of 64 rows instead, with the weights staged through LDS,
 // streams at about half the rate), and the lane holds exactly its B operands
@@ -764,9 +633,10 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
                                                          void *__restrict__ out, int out_ld) {
     // NT column tiles of 16 per wave: a block covers 64 NT weight rows (NT = 4
     // for most batches; 1 where few tiles would leave the GPU idle).
-    constexpr int BN = 64 * NT, G = KG, NSS = KG / 4;
-    static_assert(KG % 4 == 0 && KG >= 8 && KG <= STREAM_MAX_G, "whole supersteps of four groups");
-    static_assert(NT == 1 || NT == 2 || NT == 4, "1, 2 or 4 column tiles per wave");
+    constexpr int BN = 64 * NT, G = KG, NSS = (KG + 3) / 4;
+    constexpr bool HALF = KG % 4 == 2;  // the last superstep has two groups
+    static_assert(KG % 2 == 0 && KG >= 2 && KG <= STREAM_MAX_G, "an even number of groups");
+    static_assert(NT == 2 || NT == 4, "2 or 4 column tiles per wave");
     (void)K;
     (void)N;
     int tau, cb;
@@ -788,9 +658,11 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
         asrc = A + (arow * G * 2 + hl) * 64 + part * 8;
     }
     // Group j of superstep S goes to 256 j of the superstep's half.
+    auto groups_of = [](int S) { return HALF && S == NSS - 1 ? 2 : 4; };
     auto issue_a = [&](v4u *half, int S) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) dma16(asrc + (int64_t)(4 * S + j) * 128, &half[256 * j + 64 * wave]);
+        for (int j = 0; j < 4; j++)
+            if (j < groups_of(S)) dma16(asrc + (int64_t)(4 * S + j) * 128, &half[256 * j + 64 * wave]);
     };
     // Byte offsets from the block's blob (32 bits: a blob is under 4 GiB),
     // so the loads take the blob address from scalar registers.
@@ -802,47 +674,61 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
         boff[nt] = n * (G * 16) + kq * 16;
         soff[nt] = n * (G * 2) + kq * 2;
     }
+    // (a superstep of two groups: group kq / 2 instead of kq)
     auto load_b = [&](v4u (&b)[NT], int S) {
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) b[nt] = *(const v4u *)(bcodes + boff[nt] + S * 64);
+        for (int nt = 0; nt < NT; nt++) {
+            const uint32_t at = groups_of(S) == 4 ? boff[nt] : boff[nt] - (uint32_t)(kq - (kq >> 1)) * 16;
+            b[nt] = *(const v4u *)(bcodes + at + S * 64);
+        }
     };
     auto load_s = [&](uint32_t (&s)[NT], int S) {
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) s[nt] = *(const uint16_t *)(bscales + soff[nt] + S * 8);
+        for (int nt = 0; nt < NT; nt++) {
+            const uint32_t at = groups_of(S) == 4 ? soff[nt] : soff[nt] - (uint32_t)(kq - (kq >> 1)) * 2;
+            s[nt] = *(const uint16_t *)(bscales + at + S * 8);
+        }
     };
 
     const PairMagic magic = pair_magic();
     float4v acc[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) acc[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
-    auto compute = [&](const v4u *half, const v4u (&b)[NT], const uint32_t (&s)[NT]) {
+    auto compute = [&](const v4u *half, const v4u (&b)[NT], const uint32_t (&s)[NT], int S) {
         half2v scale[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
             const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)s[nt]);
             scale[nt] = (half2v){sh, sh};
         }
-        const v4u *ag = half + 256 * kq;  // the lane's group of the superstep
+        // A superstep of four groups: lane quarter kq takes group kq, part t
+        // of it in step t. One of two groups: quarter kq takes half kq % 2 of
+        // group kq / 2, in four steps.
+        const bool four = groups_of(S) == 4;
+        const v4u *ag = half + 256 * (four ? kq : kq >> 1);
+        const bool second = (kq & 1) != 0;
 #pragma unroll
         for (int t = 0; t < 8; t++) {
-            const int slot = t ^ ((col >> 1) & 7);
+            if (!four && t >= 4) break;
+            const int slot = (four ? t : 4 * (kq & 1) + t) ^ ((col >> 1) & 7);
             const half8 ahi = __builtin_bit_cast(half8, ag[col * 8 + slot]);
             const half8 alo = __builtin_bit_cast(half8, ag[(16 + col) * 8 + slot]);
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
-                const uint32_t w = (t >> 1) == 0 ? b[nt].x : (t >> 1) == 1 ? b[nt].y : (t >> 1) == 2 ? b[nt].z : b[nt].w;
+                const uint32_t w = four ? ((t >> 1) == 0 ? b[nt].x : (t >> 1) == 1 ? b[nt].y : (t >> 1) == 2 ? b[nt].z : b[nt].w)
+                                        : ((t >> 1) == 0 ? (second ? b[nt].z : b[nt].x) : (second ? b[nt].w : b[nt].y));
                 const half8 bb = b_operand_word(w >> (8 * (t & 1)), magic, scale[nt]);
                 acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bb, acc[nt], 0, 0, 0);
                 acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb, acc[nt], 0, 0, 0);
             }
         }
     };
-    // Superstep S in flight: 4 DMAs, NT code loads, NT scale loads per
+    // Superstep S in flight: a DMA a group, NT code loads, NT scale loads per
     // thread, issued in that order, all of S before any of S + 1 (memory
     // fences between the supersteps: the waits count loads in issue order).
     // Three slots: superstep S + 2 is issued into the slot of S - 1 once
     // every wave has passed the barrier that starts S.
-    constexpr int PER_SS = 4 + 2 * NT;
+    constexpr int PER_SS = 4 + 2 * NT, PER_LAST = (HALF ? 2 : 4) + 2 * NT;
     v4u b0[NT], b1[NT], b2[NT];
     uint32_t s0[NT], s1[NT], s2[NT];
     auto issue = [&](int S) {
@@ -867,20 +753,21 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
     for (int S = 0; S < NSS; S++) {
         // Superstep S complete for this wave (S + 1 may stay in flight),
         // then for every wave.
-        if (S + 1 < NSS) ring_sync<PER_SS>();
+        if (S + 2 < NSS) ring_sync<PER_SS>();
+        else if (S + 1 < NSS) ring_sync<PER_LAST>();
         else ring_sync<0>();
         if (S + 2 < NSS) issue(S + 2);
         // The unpacking of the superstep's codes stays behind the wait (the
         // compiler would otherwise start it early and wait for every load).
         if (S % 3 == 0) {
             pin_operands(b0, s0);
-            compute(g_rows16_0, b0, s0);
+            compute(g_rows16_0, b0, s0, S);
         } else if (S % 3 == 1) {
             pin_operands(b1, s1);
-            compute(g_rows16_1, b1, s1);
+            compute(g_rows16_1, b1, s1, S);
         } else {
             pin_operands(b2, s2);
-            compute(g_rows16_2, b2, s2);
+            compute(g_rows16_2, b2, s2, S);
         }
     }
 
@@ -992,6 +879,31 @@ inline uint64_t big_tile_bound(uint64_t m, int experts) {
     return m / 64 + std::min((uint64_t)experts + 1, m / 33) + 1;
 }
 
+// The streaming kernels by product and group count (stream_groups).
+using StreamKernel = decltype(&k_moe_gemm_stream<true, 2, 2, 8>);
+template <bool GATE_UP, int G>
+StreamKernel stream_kernel_at(int small_nt) {
+    if constexpr (stream_groups(GATE_UP, G)) {
+        return small_nt == 0                        ? k_moe_gemm_stream<GATE_UP, 2, 2, G>
+               : small_nt == kSmallBatchColumnTiles ? k_moe_gemm_rows16<GATE_UP, G, kSmallBatchColumnTiles>
+                                                    : k_moe_gemm_rows16<GATE_UP, G, 4>;
+    } else {
+        return nullptr;
+    }
+}
+template <bool GATE_UP, int... I>
+StreamKernel stream_kernel(int groups, int small_nt, std::integer_sequence<int, I...>) {
+    StreamKernel k = nullptr;
+    ((groups == 2 * (I + 1) ? (void)(k = stream_kernel_at<GATE_UP, 2 * (I + 1)>(small_nt)) : (void)0), ...);
+    return k;
+}
+// small_nt column tiles per wave of the 16-row kernel; 64-row tiles.
+StreamKernel small_kernel(bool gate_up, int groups, int small_nt) {
+    using Groups = std::make_integer_sequence<int, STREAM_MAX_G / 2>;
+    return gate_up ? stream_kernel<true>(groups, small_nt, Groups{}) : stream_kernel<false>(groups, small_nt, Groups{});
+}
+StreamKernel big_kernel(bool gate_up, int groups) { return small_kernel(gate_up, groups, 0); }
+
 struct PrefillWs {
     uint64_t logits, rcert, gate, dispatch, offsets, tiles_small, tiles_big, info_small, info_big,
         rows, parts, where_, Xhl, Hhl, P, Xn, end;
@@ -1042,14 +954,15 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
     const float *resid = nullptr;
     if ((2 * ff) % 128 || width % 128)
         return fail(ctx, SM_E_ARG, "prefill needs width and 2*ff to be multiples of 128");
-    // Streaming kernels: N a multiple of 256 and K one of the compiled group
-    // counts in both products (512, 640, 2048, 2560: the benchmark's and the
-    // real model's shapes). Every segment then runs in 16-row tiles below
+    // Streaming kernels: N a multiple of 256 and K of a compiled group count
+    // in both products. Every segment then runs in 16-row tiles below
     // kOneGridTokens tokens; from there on segments of up to 32 rows do, and
     // longer ones run in 64-row tiles. Other shapes: segments of up to 32
     // rows in one 32-row tile, longer ones in 64-row tiles (k_moe_gemm).
-    auto streamable = [](int k) { return k == 512 || k == 640 || k == 2048 || k == 2560; };
-    const bool stream = (2 * ff) % 256 == 0 && width % 256 == 0 && streamable(width) && streamable(ff);
+    // (200 tokens at width 1,024, ff 256, 64 experts, top-6, the layer:
+    // 125 us with k_moe_gemm, 46 us streaming.)
+    const bool stream = (2 * ff) % 256 == 0 && width % 256 == 0 && stream_groups(true, width / 64) &&
+                        stream_groups(false, ff / 64);
     // Streaming shapes issue the split, the router and the dispatch on the
     // library's stream: a fork to the second stream and the join back inside
     // a graph cost more than the overlap they buy (A/B on one GPU, graph
@@ -1082,39 +995,10 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
     const _Float16 *xhl = (const _Float16 *)(ws + w.Xhl), *hhl = (const _Float16 *)(ws + w.Hhl);
     const uint8_t *ar = (const uint8_t *)arena, *sh = (const uint8_t *)shared_blob;
 
-    // Streaming GEMM launchers by K: 64-row tiles, and 16-row tiles in whole
-    // supersteps of four groups where K allows (512, 2048, 2560), else one
-    // group per ring step (640).
-    using KT = decltype(&k_moe_gemm_stream<true, 2, 2, 8>);
-    auto big_kernel = [](bool gate_up, int K) -> KT {
-        const KT gu[4] = {k_moe_gemm_stream<true, 2, 2, 8>, k_moe_gemm_stream<true, 2, 2, 10>,
-                          k_moe_gemm_stream<true, 2, 2, 32>, k_moe_gemm_stream<true, 2, 2, 40>};
-        const KT dn[4] = {k_moe_gemm_stream<false, 2, 2, 8>, k_moe_gemm_stream<false, 2, 2, 10>,
-                          k_moe_gemm_stream<false, 2, 2, 32>, k_moe_gemm_stream<false, 2, 2, 40>};
-        const int kv = K == 512 ? 0 : K == 640 ? 1 : K == 2048 ? 2 : 3;
-        return gate_up ? gu[kv] : dn[kv];
-    };
-    // 16-row tiles: 256 weight rows per block, or 64 (one column tile per
+    // 16-row tiles: 256 weight rows per block, or 128 (two column tiles per
     // wave) for batches of up to kSmallBatch tokens, whose few tiles would
-    // otherwise leave most CUs idle (K = 640 always 256).
+    // otherwise leave most CUs idle.
     const int small_nt = tokens <= kSmallBatch ? kSmallBatchColumnTiles : 4;
-    auto small_kernel = [small_nt](bool gate_up, int K) -> KT {
-        const KT gu[4] = {k_moe_gemm_rows16<true, 8>, k_moe_gemm_stream16<true, 10>, k_moe_gemm_rows16<true, 32>,
-                          k_moe_gemm_rows16<true, 40>};
-        const KT dn[4] = {k_moe_gemm_rows16<false, 8>, k_moe_gemm_stream16<false, 10>, k_moe_gemm_rows16<false, 32>,
-                          k_moe_gemm_rows16<false, 40>};
-        const KT gu_n[4] = {k_moe_gemm_rows16<true, 8, kSmallBatchColumnTiles>, k_moe_gemm_stream16<true, 10>,
-                            k_moe_gemm_rows16<true, 32, kSmallBatchColumnTiles>,
-                            k_moe_gemm_rows16<true, 40, kSmallBatchColumnTiles>};
-        const KT dn_n[4] = {k_moe_gemm_rows16<false, 8, kSmallBatchColumnTiles>, k_moe_gemm_stream16<false, 10>,
-                            k_moe_gemm_rows16<false, 32, kSmallBatchColumnTiles>,
-                            k_moe_gemm_rows16<false, 40, kSmallBatchColumnTiles>};
-        const int kv = K == 512 ? 0 : K == 640 ? 1 : K == 2048 ? 2 : 3;
-        if (small_nt != 4) return gate_up ? gu_n[kv] : dn_n[kv];
-        return gate_up ? gu[kv] : dn[kv];
-    };
-    // weight rows per block of the 16-row kernel for K
-    auto small_bn = [small_nt](int K) { return K == 640 ? 256 : 64 * small_nt; };
 
     // Other shapes: the split on the second stream, beside the router.
     const bool aux = !one_stream;  // the second stream holds work from here to the combine
@@ -1191,13 +1075,13 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
             int rc_big = SM_OK;
             if (any_big) {
                 if (int rc3 = fork_aux(ctx)) return rc3;
-                big_kernel(gate_up, K)<<<dim3((unsigned)(N / 256), big_tiles), 256, 0, ctx->aux>>>(
+                big_kernel(gate_up, K / 64)<<<dim3((unsigned)(N / 256), big_tiles), 256, 0, ctx->aux>>>(
                     a, r, info_big, tiles_big, ar, blob_stride, sh, experts, codes, scales, K, N, out, ld);
                 rc_big = launched(ctx);
             }
             int rc_small = SM_OK;
             if (rc_big == SM_OK) {
-                small_kernel(gate_up, K)<<<dim3((unsigned)(N / small_bn(K)), small_tiles), 256, 0, ctx->stream>>>(
+                small_kernel(gate_up, K / 64, small_nt)<<<dim3((unsigned)(N / (64 * small_nt)), small_tiles), 256, 0, ctx->stream>>>(
                     a, r, info_small, tiles_small, ar, blob_stride, sh, experts, codes, scales, K, N, out, ld);
                 rc_small = launched(ctx);
             }
