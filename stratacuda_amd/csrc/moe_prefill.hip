@@ -172,6 +172,18 @@ __device__ __forceinline__ half8 b_operand_word(uint32_t w, const PairMagic &m, 
     const half8 b = {p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
     return b;
 }
+// The same without the scale: c - 1, two VALU operations per pair.
+template <int Q>
+__device__ __forceinline__ half2v pair_codes(uint32_t wq, const PairMagic &m) {
+    constexpr uint32_t e = 25 - 2 * Q, magic = (e << 10) | (e << 26);
+    constexpr float sub = (float)((1 << (10 - 2 * Q)) + 1);
+    return __builtin_bit_cast(half2v, and_or_b32(wq, m.mask[Q], magic)) - (half2v){(_Float16)sub, (_Float16)sub};
+}
+__device__ __forceinline__ half8 b_codes_word(uint32_t w, const PairMagic &m) {
+    const half2v p0 = pair_codes<0>(w, m), p1 = pair_codes<1>(w, m), p2 = pair_codes<2>(w, m), p3 = pair_codes<3>(w, m);
+    const half8 b = {p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y};
+    return b;
+}
 __device__ __forceinline__ half8 b_operand_stream(uint4 c, int s, uint32_t shift, const PairMagic &m,
                                                   half2v scale) {
     return b_operand_word((s == 0 ? c.x : s == 1 ? c.y : s == 2 ? c.z : c.w) >> shift, m, scale);
@@ -618,10 +630,25 @@ __shared__ __attribute__((aligned(16))) v4u g_rows16_0[4 * 256], g_rows16_1[4 * 
 
 // An empty volatile statement that reads and rewrites the registers: code
 // using them cannot move above the volatile wait before it.
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 template <int NT>
-__device__ __forceinline__ void pin_operands(v4u (&b)[NT], uint32_t (&s)[NT]) {
+__device__ __forceinline__ void pin_operands(v4u (&b)[NT], v2u (&s)[NT]) {
 #pragma unroll
     for (int i = 0; i < NT; i++) asm volatile("" : "+v"(b[i]), "+v"(s[i]));
+}
+// Transposes 4 x 4 words between the registers and the four lane quarters:
+// lane quarter k's register j becomes quarter j's register k.
+__device__ __forceinline__ v4u transpose_quarters(v4u v) {
+    const auto xz = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+    const auto yw = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+    const auto lo = __builtin_amdgcn_permlane16_swap(xz[0], yw[0], false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(xz[1], yw[1], false, false);
+    return v4u{lo[0], lo[1], hi[0], hi[1]};
+}
+// Scale of group j of a superstep: the fp16 values of four groups in 8 bytes.
+__device__ __forceinline__ float group_scale(v2u s, int j) {
+    const uint16_t h = (uint16_t)((j < 2 ? s.x : s.y) >> (16 * (j & 1)));
+    return (float)__builtin_bit_cast(_Float16, h);
 }
 
 template <bool GATE_UP, int KG, int NT = 4>
@@ -672,21 +699,31 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
     for (int nt = 0; nt < NT; nt++) {
         const uint32_t n = (uint32_t)(n0 + wave * 16 * NT + nt * 16 + col);
         boff[nt] = n * (G * 16) + kq * 16;
-        soff[nt] = n * (G * 2) + kq * 2;
+        soff[nt] = n * (G * 2);
     }
-    // (a superstep of two groups: group kq / 2 instead of kq)
+    // Four groups: the 16 code bytes of the lane's own. Two: word kq of each.
     auto load_b = [&](v4u (&b)[NT], int S) {
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            const uint32_t at = groups_of(S) == 4 ? boff[nt] : boff[nt] - (uint32_t)(kq - (kq >> 1)) * 16;
-            b[nt] = *(const v4u *)(bcodes + at + S * 64);
+            if (groups_of(S) == 4) {
+                b[nt] = *(const v4u *)(bcodes + boff[nt] + S * 64);
+            } else {
+                const uint8_t *p = bcodes + (boff[nt] - (uint32_t)kq * 12) + S * 64;
+                b[nt].x = *(const uint32_t *)p;
+                b[nt].y = *(const uint32_t *)(p + 16);
+            }
         }
     };
-    auto load_s = [&](uint32_t (&s)[NT], int S) {
+    // the scales of the superstep's groups (rows start 4-byte aligned)
+    auto load_s = [&](v2u (&s)[NT], int S) {
+        struct __attribute__((packed, aligned(4))) Scales {
+            v2u v;
+        };
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) {
-            const uint32_t at = groups_of(S) == 4 ? soff[nt] : soff[nt] - (uint32_t)(kq - (kq >> 1)) * 2;
-            s[nt] = *(const uint16_t *)(bscales + at + S * 8);
+            const uint8_t *p = bscales + soff[nt] + S * 8;
+            if (groups_of(S) == 4) s[nt] = ((const Scales *)p)->v;
+            else s[nt].x = *(const uint32_t *)p;
         }
     };
 
@@ -694,33 +731,44 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
     float4v acc[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) acc[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
-    auto compute = [&](const v4u *half, const v4u (&b)[NT], const uint32_t (&s)[NT], int S) {
-        half2v scale[NT];
+    // Group by group, two MFMA steps each: lane quarter kq holds word kq of the
+    // group, step t takes byte half t of it and part 2 kq + t of the A row.
+    // The group's products are summed over whole codes c - 1 and its scale,
+    // one per column and so one per lane, goes on in f32.
+    auto compute = [&](const v4u *half, const v4u (&b)[NT], const v2u (&s)[NT], int S) {
+        v4u words[NT];
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)s[nt]);
-            scale[nt] = (half2v){sh, sh};
-        }
-        // A superstep of four groups: lane quarter kq takes group kq, part t
-        // of it in step t. One of two groups: quarter kq takes half kq % 2 of
-        // group kq / 2, in four steps.
-        const bool four = groups_of(S) == 4;
-        const v4u *ag = half + 256 * (four ? kq : kq >> 1);
-        const bool second = (kq & 1) != 0;
+        for (int nt = 0; nt < NT; nt++) words[nt] = groups_of(S) == 4 ? transpose_quarters(b[nt]) : b[nt];
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            if (!four && t >= 4) break;
-            const int slot = (four ? t : 4 * (kq & 1) + t) ^ ((col >> 1) & 7);
-            const half8 ahi = __builtin_bit_cast(half8, ag[col * 8 + slot]);
-            const half8 alo = __builtin_bit_cast(half8, ag[(16 + col) * 8 + slot]);
+        for (int j = 0; j < 4; j++) {
+            if (j >= groups_of(S)) break;
+            const v4u *ag = half + 256 * j;
+            float4v sum[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) sum[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int slot = (2 * kq + t) ^ ((col >> 1) & 7);
+                const half8 ahi = __builtin_bit_cast(half8, ag[col * 8 + slot]);
+                const half8 alo = __builtin_bit_cast(half8, ag[(16 + col) * 8 + slot]);
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++) {
+                    const uint32_t w = j == 0 ? words[nt].x : j == 1 ? words[nt].y : j == 2 ? words[nt].z : words[nt].w;
+                    const half8 bb = b_codes_word(w >> (8 * t), magic);
+                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bb, sum[nt], 0, 0, 0);
+                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb, sum[nt], 0, 0, 0);
+                }
+            }
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
-                const uint32_t w = four ? ((t >> 1) == 0 ? b[nt].x : (t >> 1) == 1 ? b[nt].y : (t >> 1) == 2 ? b[nt].z : b[nt].w)
-                                        : ((t >> 1) == 0 ? (second ? b[nt].z : b[nt].x) : (second ? b[nt].w : b[nt].y));
-                const half8 bb = b_operand_word(w >> (8 * (t & 1)), magic, scale[nt]);
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bb, acc[nt], 0, 0, 0);
-                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb, acc[nt], 0, 0, 0);
+                const float scale = group_scale(s[nt], j);
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[nt][i] = fmaf(sum[nt][i], scale, acc[nt][i]);
             }
+            // (the groups' sums do not depend on each other: without a line
+            // here the compiler keeps them all to the end, and spills)
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) asm volatile("" : "+v"(acc[nt]));
         }
     };
     // Superstep S in flight: a DMA a group, NT code loads, NT scale loads per
@@ -728,9 +776,9 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
     // fences between the supersteps: the waits count loads in issue order).
     // Three slots: superstep S + 2 is issued into the slot of S - 1 once
     // every wave has passed the barrier that starts S.
-    constexpr int PER_SS = 4 + 2 * NT, PER_LAST = (HALF ? 2 : 4) + 2 * NT;
+    constexpr int PER_SS = 4 + 2 * NT, PER_LAST = HALF ? 2 + 3 * NT : PER_SS;
     v4u b0[NT], b1[NT], b2[NT];
-    uint32_t s0[NT], s1[NT], s2[NT];
+    v2u s0[NT], s1[NT], s2[NT];
     auto issue = [&](int S) {
         if (S % 3 == 0) {
             issue_a(g_rows16_0, S);
