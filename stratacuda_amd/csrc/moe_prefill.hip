@@ -735,6 +735,16 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
     // group, step t takes byte half t of it and part 2 kq + t of the A row.
     // The group's products are summed over whole codes c - 1 and its scale,
     // one per column and so one per lane, goes on in f32.
+    //
+    // PACK: a tile of up to eight rows puts their hi halves in rows 0-7 of the A
+    // operand and their lo halves in rows 8-15, one MFMA for both; the two are
+    // added at the end. For the batches whose experts mostly hold that few
+    // (the narrow tiles'); with four column tiles the second path costs more
+    // registers and code than it saves (512 tokens 196 -> 225 us).
+    constexpr bool PACK = NT == 2;
+    const bool packed = PACK && mend - m0 <= 8;
+    const int arow = packed ? col & 7 : col;
+    const int first = (packed ? (col >> 3) * 16 + arow : arow) * 8, second = (16 + arow) * 8;
     auto compute = [&](const v4u *half, const v4u (&b)[NT], const v2u (&s)[NT], int S) {
         v4u words[NT];
 #pragma unroll
@@ -744,19 +754,30 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
             if (j >= groups_of(S)) break;
             const v4u *ag = half + 256 * j;
             float4v sum[NT];
+            half8 bb[2][NT];
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) sum[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+            auto part = [&](int at, int t) { return __builtin_bit_cast(half8, ag[at + ((2 * kq + t) ^ ((arow >> 1) & 7))]); };
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                const int slot = (2 * kq + t) ^ ((col >> 1) & 7);
-                const half8 ahi = __builtin_bit_cast(half8, ag[col * 8 + slot]);
-                const half8 alo = __builtin_bit_cast(half8, ag[(16 + col) * 8 + slot]);
+                const half8 ahi = part(first, t);
+                half8 alo;
+                if (!PACK) alo = part(second, t);
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++) {
                     const uint32_t w = j == 0 ? words[nt].x : j == 1 ? words[nt].y : j == 2 ? words[nt].z : words[nt].w;
-                    const half8 bb = b_codes_word(w >> (8 * t), magic);
-                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bb, sum[nt], 0, 0, 0);
-                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb, sum[nt], 0, 0, 0);
+                    bb[t][nt] = b_codes_word(w >> (8 * t), magic);
+                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bb[t][nt], sum[nt], 0, 0, 0);
+                    if (!PACK) sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb[t][nt], sum[nt], 0, 0, 0);
+                }
+            }
+            if (PACK && !packed) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const half8 alo = part(second, t);
+#pragma unroll
+                    for (int nt = 0; nt < NT; nt++)
+                        sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb[t][nt], sum[nt], 0, 0, 0);
                 }
             }
 #pragma unroll
@@ -819,10 +840,22 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
         }
     }
 
+    // Packed: row r's hi sum is in lane quarter r / 4, its lo sum two quarters on.
+    if (packed) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const auto lo = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[nt][i]), __float_as_uint(acc[nt][i]),
+                                                                 false, false);
+                acc[nt][i] = acc[nt][i] + __uint_as_float(lo[1]);
+            }
+    }
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
+            // (packed: the quarters past row 7 fall past the segment's end)
             const int pos = m0 + 4 * kq + i, n = n0 + wave * 16 * NT + nt * 16 + col;
             if (GATE_UP) {
                 const float other = sm::dpp_f32<sm::kDppQuadXor1>(acc[nt][i], acc[nt][i]);
@@ -910,8 +943,13 @@ inline uint64_t up(uint64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 // tokens 0.372 -> 0.415 ms; with uniform routing 0.373 -> 0.365 and 0.460 ->
 // 0.465 ms.)
 constexpr int kOneGridTokens = 1024;
-constexpr int kSmallBatch = 64;
-constexpr int kSmallBatchColumnTiles = 2;  // column tiles per wave of the 16-row kernel up to kSmallBatch tokens
+// Column tiles per wave of the 16-row kernel: two up to kSmallBatch tokens,
+// where the few tiles would leave CUs idle and most hold up to eight rows
+// (packed tiles), four above. Four against two, us a layer: 65 tokens 128.3 /
+// 122.8, 128 161 / 156, 200 177 / 174, 333 at 2560 / 640 288 / 282, 512 196 /
+// 199.
+constexpr int kSmallBatch = 384;
+constexpr int kSmallBatchColumnTiles = 2;
 inline int tiling_split(int tokens) { return tokens < kOneGridTokens ? tokens + 1 : 33; }
 
 // Grid bounds of the two tilings over the experts + 1 segments of m rows:
@@ -1043,9 +1081,7 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
     const _Float16 *xhl = (const _Float16 *)(ws + w.Xhl), *hhl = (const _Float16 *)(ws + w.Hhl);
     const uint8_t *ar = (const uint8_t *)arena, *sh = (const uint8_t *)shared_blob;
 
-    // 16-row tiles: 256 weight rows per block, or 128 (two column tiles per
-    // wave) for batches of up to kSmallBatch tokens, whose few tiles would
-    // otherwise leave most CUs idle.
+    // 16-row tiles: 256 weight rows per block, or 128 up to kSmallBatch tokens.
     const int small_nt = tokens <= kSmallBatch ? kSmallBatchColumnTiles : 4;
 
     // Other shapes: the split on the second stream, beside the router.
