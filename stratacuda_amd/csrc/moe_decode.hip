@@ -342,13 +342,16 @@ __global__ void __launch_bounds__(256) k_decode_route(const float *__restrict__ 
     }
 }
 
-// K2. Grid (ceil(ff / 16), topk + 1). Slot blockIdx.y < topk: wave 0 runs the
+// K2. Grid (ceil(ff / (16 REPS)), topk + 1, tokens). Slot blockIdx.y < topk: wave 0 runs the
 // top-k into LDS (block (0,0) also writes ids / weights to memory), then every
 // wave computes 4 hidden rows of that routed expert. Slot topk is the shared
 // expert and needs no routing.
 // EXTRA: 33-40 groups per row (the real model's 2560), whose groups 32..
 // are spread one (row, group) pair per lane.
-template <bool EXTRA>
+//
+// REPS: a wave computes that many times GU_ROWS rows with one read of its
+// activation records (200 bytes a lane, against 64 of codes for four rows).
+template <bool EXTRA, int REPS>
 __global__ void __launch_bounds__(256) k_decode_gate_up(const uint32_t *__restrict__ xq,
                                                         const uint8_t *__restrict__ arena, uint64_t stride,
                                                         const uint8_t *__restrict__ shared_blob,
@@ -388,9 +391,12 @@ __global__ void __launch_bounds__(256) k_decode_gate_up(const uint32_t *__restri
     }
     __syncthreads();
     const uint8_t *blob = slot_blob(arena, stride, shared_blob, k < topk ? s_ids[k] : 0, k, topk, experts);
-    const int j0 = (blockIdx.x * GU_WAVES + wave) * GU_ROWS;
-    if (j0 < ff)
-        gate_up_rows<EXTRA>(xq, first, second, blob, gu_scales, hidden + (uint64_t)k * ff, j0, width, ff, s_tab);
+    const int j0 = (blockIdx.x * GU_WAVES + wave) * GU_ROWS * REPS;
+#pragma unroll
+    for (int rep = 0; rep < REPS; rep++)
+        if (j0 + GU_ROWS * rep < ff)
+            gate_up_rows<EXTRA>(xq, first, second, blob, gu_scales, hidden + (uint64_t)k * ff, j0 + GU_ROWS * rep, width,
+                                ff, s_tab);
     // Block (0, 0) publishes the token's IDs and routing weights, after its
     // own expert work so that no block's loads wait for the weights.
     if (k == 0 && !routed && blockIdx.x == 0 && wave == 0) {
@@ -930,7 +936,7 @@ __device__ uint64_t g_fused_trace[kFusedBlocks * 32];
 // W x F: hidden 2048 / ff 512 (the benchmark geometry) or hidden 2560 / ff
 // 640 (the real model's, RG below). RG differs in three places: 40 groups
 // per gate/up row (groups 32-39 spread one (row, group) pair per lane, as
-// in k_decode_gate_up<true>), 7,040 hidden rows (waves 0-3 of a block take
+// in k_decode_gate_up<true, 1>), 7,040 hidden rows (waves 0-3 of a block take
 // four, waves 4-7 three: at most seven per SIMD), and 10 output rows per
 // block whose 1,100 (slot, row, group) down products are spread over the
 // block's threads with every slot's hidden vector in LDS, summed per row in
@@ -1167,7 +1173,7 @@ __global__ void __launch_bounds__(64 * kFusedWaves, 1) k_decode_fused(FusedArgs 
     const int nrow = RG ? (wave < 4 ? 4 : 3) : kFusedRows;
     const int base = RG ? b * RG_ITEMS + (wave < 4 ? 4 * wave : 16 + 3 * (wave - 4)) : gw * kFusedRows;
     // RG: the lane's (row, group) pair of groups 32-39: group g2 of the
-    // wave's row r2 whose item is gl / 8 modulo 4. k_decode_gate_up<true>
+    // wave's row r2 whose item is gl / 8 modulo 4. k_decode_gate_up<true, 1>
     // gives item i's pairs to lanes 8 (i % 4) .. + 7 (its waves start at
     // multiples of 4), and the lane a product lands on fixes the rounding of
     // the half-wave sum; a wave's rows are at most 4 consecutive items, so
@@ -1221,7 +1227,7 @@ __global__ void __launch_bounds__(64 * kFusedWaves, 1) k_decode_fused(FusedArgs 
         FUSED_MARK_LOADED(16 + wave);
         float acc[RB];
         if constexpr (RG) {
-            // k_decode_gate_up<true>'s sums: group gl by fma onto 0, then the
+            // k_decode_gate_up<true, 1>'s sums: group gl by fma onto 0, then the
             // pair's product added to its row (and +0 to the others)
 #pragma unroll
             for (int r = 0; r < RB; r++) acc[r] = fmaf(sm::half_bits(sb[r]), dot64_q(c[r], xq), 0.0f);
@@ -1726,9 +1732,16 @@ int moe_decode(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias, 
             return rc;
     if (stage_on(ctx, kStageDecodeGateUp)) {
         if (int rc = stage_mark(ctx, kStageDecodeGateUp)) return rc;
-        dim3 g1((unsigned)blocks_per_expert, (unsigned)(topk + 1), (unsigned)tokens);
+        // Twice the rows per wave once the grid has two blocks a CU without:
+        // four stack blocks of 4 tokens 133 -> 121 us, 5 162 -> 153, 6 179 ->
+        // 170, 2 at 2560 / 640 152 -> 136; a smaller grid loses (3 tokens of a
+        // 256-row expert, 336 blocks, 71 -> 73). Four times: 128, 150, 176, 137.
+        const int reps = (int64_t)blocks_per_expert * (topk + 1) * tokens <= 512 ? 1 : 2;
+        dim3 g1((unsigned)ceil_div(blocks_per_expert, reps), (unsigned)(topk + 1), (unsigned)tokens);
         const int G = width / 64;
-        const auto k2 = G > 32 && G <= 40 ? k_decode_gate_up<true> : k_decode_gate_up<false>;
+        const bool extra = G > 32 && G <= 40;
+        const auto k2 = reps == 1 ? (extra ? k_decode_gate_up<true, 1> : k_decode_gate_up<false, 1>)
+                                  : (extra ? k_decode_gate_up<true, 2> : k_decode_gate_up<false, 2>);
         k2<<<g1, 64 * GU_WAVES, 0, ctx->stream>>>(
             xq, (const uint8_t *)arena, blob_stride, (const uint8_t *)shared_blob, (const float *)(ws + w.logits),
             (int *)ids, (float *)weights, hidden, width, ff, topk, experts, L.gate_up_scales, routed);
