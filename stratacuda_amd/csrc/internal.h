@@ -236,6 +236,11 @@ bool project_batch_takes(int bits, int cols, int tokens, uint64_t X, uint64_t co
 int project_batch(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets,
                   float *Y, int cols, int rows, int tokens, int stride, int out, int group, int bias, int codebook,
                   int has_offset);
+// The same of one token, quantized codes only (strata_quant_gemv).
+bool project_one_takes(int bits, int cols, uint64_t X, uint64_t codes, uint64_t scales, uint64_t offsets, int group, int bias,
+                       int codebook);
+int project_one(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets, float *Y,
+                int cols, int rows, int group, int bias, int codebook, int has_offset);
 
 // ------------------------------------------------ kernels by name (sm_run)
 // One 64-bit slot per reference parameter: a buffer handle, or the int32 /

@@ -1,6 +1,7 @@
-// Dense projections of a token batch (strata_bf16_project and
+// Dense projections. A token batch (strata_bf16_project and
 // strata_quant_project with two or more tokens): every weight is read and
-// widened once for up to 16 tokens, with the reference's sums.
+// widened once for up to 16 tokens, with the reference's sums. One token of
+// quantized weights: k_project_one below.
 //
 // The reference's order (kernels/strata.cu:156-165) is 64 partial sums per
 // output, partial p over the columns p, p + 64, ... one rounded product and
@@ -231,6 +232,88 @@ __global__ void __launch_bounds__(256, 2) k_project_batch(ProjectArgs a) {
     }
 }
 
+// strata_quant_gemv (kernels/strata.cu:134-155: strata_quant_project's
+// arithmetic for one token). The same lanes as above, with the products on
+// the vector unit: a wave owns four rows, lane l the columns 4 (l / 4) .. + 3
+// of every step for row l % 4. The wave's codes, scales and offsets and the
+// block's copy of x all arrive by DMA at once, and the steps run from LDS:
+// four weights for a code, a scale, an offset and a 16-byte x read, where one
+// weight a lane cost three reads. Code rows lie 2 BITS words apart modulo 32,
+// so that the four rows of a step meet different banks. Bound: the vector
+// instructions (seven a weight) and the stream about equally. 2,560 x 10,240
+// with 32-weight groups and offsets, from a graph, us: 4 bits 13.7 -> 10.4, 8
+// bits 20.1 -> 14.6; 3,072 x 300 at 8 bits 11.2 -> 7.7.
+constexpr uint64_t kOneTokenLds = 65536;
+__host__ __device__ constexpr int one_token_pitch(int bits, int cols) {
+    const int words = cols * bits / 32;
+    return words + (2 * bits + 32 - words % 32) % 32;
+}
+template <int BITS, bool CODEBOOK>
+__global__ void __launch_bounds__(256) k_project_one(ProjectArgs a) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t s_one[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int b = lane >> 2, i = lane & 3, steps = a.cols >> 6;
+    const int words = a.cols * BITS / 32, pitch = one_token_pitch(BITS, a.cols), ng = a.cols >> a.group_shift;
+    float *s_x = (float *)s_one;
+    uint32_t *codes = s_one + a.cols + wave * 4 * (pitch + 2 * ng);
+    float *scales = (float *)(codes + 4 * pitch), *offsets = scales + 4 * ng;
+    const int r0 = (blockIdx.x * waves + wave) * 4, nr = min(4, a.rows - r0);
+    for (int c = 256 * wave; c < a.cols; c += 256 * waves)
+        if (c + 4 * lane < a.cols)
+            __builtin_amdgcn_global_load_lds(a.X + c + 4 * lane, (lds_void_t *)(s_x + c), 16, 0, 0);
+    for (int r = 0; r < nr; r++) {
+        const uint8_t *row = a.codes + (int64_t)(r0 + r) * words * 4;
+        for (int c = 0; c < words; c += 256)
+            if (c + 4 * lane < words)
+                __builtin_amdgcn_global_load_lds(row + 4 * (c + 4 * lane), (lds_void_t *)(codes + r * pitch + c), 16, 0, 0);
+    }
+    // (four rows' groups are whole 16-byte pieces, fewer rows' may not be)
+    auto groups = [&](const float *src, float *dst) {
+        src += (int64_t)r0 * ng;
+        if (nr == 4) {
+            for (int c = 0; c < 4 * ng; c += 256)
+                if (c + 4 * lane < 4 * ng)
+                    __builtin_amdgcn_global_load_lds(src + c + 4 * lane, (lds_void_t *)(dst + c), 16, 0, 0);
+        } else {
+            for (int c = 0; c < nr * ng; c += 64)
+                if (c + lane < nr * ng) __builtin_amdgcn_global_load_lds(src + c + lane, (lds_void_t *)(dst + c), 4, 0, 0);
+        }
+    };
+    groups(a.scales, scales);
+    if (a.has_offset) groups(a.offsets, offsets);
+    __builtin_amdgcn_s_waitcnt(0 | 0x7 << 4 | 0xF << 8);  // vmcnt(0)
+    __syncthreads();
+    if (nr < 1) return;
+    const int row = min(i, nr - 1);
+    const uint8_t *code = (const uint8_t *)(codes + row * pitch) + b * BITS / 2;
+    const float *sc = scales + row * ng, *of = (a.has_offset ? offsets : scales) + row * ng, *x = s_x + 4 * b;
+    float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int k = 0; k < steps; k++) {
+        Raw<BITS> raw;
+        const uint8_t *c = code + k * 8 * BITS;
+        raw.code[0] = BITS == 8 ? *(const uint32_t *)c : BITS == 4 ? *(const uint16_t *)c : *c;
+        const int g = (64 * k + 4 * b) >> a.group_shift;
+        raw.scale = sc[g];
+        raw.offset = of[g];
+        const f32x4 xv = *(const f32x4 *)(x + 64 * k);
+        float w[4];
+        widen<BITS, CODEBOOK>(a, raw, w);
+#pragma unroll
+        for (int q = 0; q < 4; q++) sum[q] = sum[q] + w[q] * xv[q];
+    }
+    // the reference's tree: columns 32, 16, 8 and 4 apart are lanes, 2 and 1 are q
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        float v = sum[q];
+        v = v + __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false)[1]);
+        v = v + __uint_as_float(__builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false)[1]);
+        v = v + sm::dpp_f32<0x108>(0.0f, v);
+        sum[q] = v + sm::dpp_f32<0x104>(0.0f, v);
+    }
+    if (lane < nr) a.Y[r0 + lane] = (sum[0] + sum[2]) + (sum[1] + sum[3]);
+}
+
 template <int BITS, bool CODEBOOK>
 void launch(sm_ctx *ctx, const ProjectArgs &a, int ng) {
     const dim3 grid((unsigned)((a.rows + 15) / 16), (unsigned)((a.tokens + 4 * ng - 1) / (4 * ng)));
@@ -281,6 +364,31 @@ int project_batch(sm_ctx *ctx, int bits, const float *X, const void *codes, cons
         case 8: launch<8, false>(ctx, a, ng); break;
         default: launch<16, false>(ctx, a, ng); break;
     }
+    return launched(ctx);
+}
+
+// LDS of a block of `waves` waves.
+static uint64_t one_token_lds(int bits, int cols, int group, int waves) {
+    return 4ull * (cols + (uint64_t)waves * 4 * (one_token_pitch(bits, cols) + 2 * (cols / group)));
+}
+
+bool project_one_takes(int bits, int cols, uint64_t X, uint64_t codes, uint64_t scales, uint64_t offsets, int group, int bias,
+                       int codebook) {
+    if (cols % 64 || (X | codes | scales | offsets) % 16) return false;
+    if (group < 4 || (group & (group - 1)) || (codebook == 1 && bits != 4)) return false;
+    return bias > -(1 << 23) && bias < (1 << 23) - 256 && one_token_lds(bits, cols, group, 1) <= kOneTokenLds;
+}
+
+int project_one(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets, float *Y,
+                int cols, int rows, int group, int bias, int codebook, int has_offset) {
+    ProjectArgs a = {X, (const uint8_t *)codes, scales, offsets, Y, cols, rows, 1, rows, 0, 0, has_offset, (float)bias};
+    while ((1 << a.group_shift) < group) a.group_shift++;
+    int waves = 4;
+    while (one_token_lds(bits, cols, group, waves) > kOneTokenLds) waves--;
+    const auto k = bits == 2   ? k_project_one<2, false>
+                   : bits == 8 ? k_project_one<8, false>
+                               : (codebook == 1 ? k_project_one<4, true> : k_project_one<4, false>);
+    k<<<(unsigned)((rows + 4 * waves - 1) / (4 * waves)), 64 * waves, one_token_lds(bits, cols, group, waves), ctx->stream>>>(a);
     return launched(ctx);
 }
 

@@ -68,3 +68,27 @@ def test_quant_batch(backend, oracle, cols, rows, tokens, nbits, group, codebook
     want = oracle.quant_project(x, codes, scales, offsets, np.full(tokens * stride, -7, np.float32), cols, rows, tokens,
                                 stride, off, nbits, group, bias, codebook, offset)
     same(backend.read(y), want)
+
+
+@pytest.mark.parametrize("cols,rows", [(64, 1), (128, 3), (320, 17), (2560, 4100), (4096, 66), (3072, 301), (100, 7)])
+@pytest.mark.parametrize("nbits,group,codebook,offset", [(4, 32, 0, 1), (8, 32, 0, 1), (4, 64, 1, 0), (2, 4, 0, 0),
+                                                         (8, 64, 0, 0), (2, 32, 0, 1), (4, 2, 0, 1)])
+def test_quant_one_token(backend, oracle, cols, rows, nbits, group, codebook, offset):
+    """One token: blocks of four, three and fewer waves (the rows' bytes in LDS), waves of four rows and fewer."""
+    if cols % group:
+        group = 4
+    rng, x = inputs(cols, rows, 2)
+    x = x[:cols] if rows % 2 else x[cols:]
+    codes = rng.integers(0, 1 << 32, (rows * cols * nbits + 31) // 32, dtype=np.uint32)
+    scales = rng.normal(0, 0.02, rows * cols // group).astype(np.float32)
+    offsets = rng.normal(0, 0.01, scales.size).astype(np.float32)
+    bias = -(1 << (nbits - 1))
+    y = backend.alloc(np.full(rows + 1, -7, np.float32))
+    backend.run("strata_quant_gemv",
+                {"X": backend.alloc(x), "Codes": backend.alloc(codes, "u32"), "Scales": backend.alloc(scales),
+                 "Offsets": backend.alloc(offsets), "Y": y, "cols": cols, "rows": rows, "bits": nbits, "groupSize": group,
+                 "bias": bias, "codebook": codebook, "hasOffset": offset}, [rows, 1, 1])
+    want = oracle.quant_gemv(x, codes, scales, offsets, cols, rows, nbits, group, bias, codebook, offset)
+    got = backend.read(y)
+    same(got[:rows], np.asarray(want, np.float32).reshape(-1)[:rows])
+    assert got[rows] == -7
