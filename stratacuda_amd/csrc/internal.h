@@ -236,6 +236,10 @@ bool project_batch_takes(int bits, int cols, int tokens, uint64_t X, uint64_t co
 int project_batch(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets,
                   float *Y, int cols, int rows, int tokens, int stride, int out, int group, int bias, int codebook,
                   int has_offset);
+// Router logits of a token batch, and the shared-expert gate's with gate_w.
+bool route_batch_takes(const float *X, int width, const float *Wr, const float *gate_w);
+int route_batch(sm_ctx *ctx, const float *X, int tokens, int width, const float *Wr, const float *bias, int experts,
+                float *logits, const float *gate_w, float *gate_out);
 // The same of one token, quantized codes only (strata_quant_gemv).
 bool project_one_takes(int bits, int cols, uint64_t X, uint64_t codes, uint64_t scales, uint64_t offsets, int group, int bias,
                        int codebook);

@@ -45,7 +45,7 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 // The raw weights of one lane and one step: four columns of one row.
 template <int BITS>
 struct Raw {
-    uint32_t code[BITS == 16 ? 2 : 1];
+    uint32_t code[BITS == 32 ? 4 : BITS == 16 ? 2 : 1];
     float scale, offset;
 };
 
@@ -57,6 +57,10 @@ struct ProjectArgs {
     int cols, rows, tokens, stride, out;
     int group_shift, has_offset;
     float bias;
+    // the router (f32 weights): its last row and that row's outputs when there
+    // is a shared-expert gate, and the experts' biases
+    const float *gate_row, *expert_bias;
+    float *gate_out;
 };
 
 // IQ4_NL values (kernels/strata.cu:22-31) as signed bytes, four to a word.
@@ -67,10 +71,16 @@ constexpr uint32_t iq4_word(int a, int b, int c, int d) {
 template <int BITS>
 __device__ __forceinline__ void load_raw(const ProjectArgs &a, const uint8_t *row_codes, const float *row_scales,
                                          const float *row_offsets, int col, Raw<BITS> &w) {
-    if (BITS == 16) {
+    if constexpr (BITS == 32) {
+        const uint4 v = *(const uint4 *)(row_codes + 4 * col);
+        w.code[0] = v.x;
+        w.code[1] = v.y;
+        w.code[2] = v.z;
+        w.code[3] = v.w;
+    } else if constexpr (BITS == 16) {
         const uint2 v = *(const uint2 *)(row_codes + 2 * col);
         w.code[0] = v.x;
-        w.code[BITS == 16 ? 1 : 0] = v.y;
+        w.code[1] = v.y;
     } else {
         if (BITS == 8) w.code[0] = *(const uint32_t *)(row_codes + col);
         if (BITS == 4) w.code[0] = *(const uint16_t *)(row_codes + col / 2);
@@ -86,11 +96,15 @@ __device__ __forceinline__ void load_raw(const ProjectArgs &a, const uint8_t *ro
 // no partial sum tells a product of -0 from one of +0.
 template <int BITS, bool CODEBOOK>
 __device__ __forceinline__ void widen(const ProjectArgs &a, const Raw<BITS> &w, float (&out)[4]) {
-    if (BITS == 16) {
+    if constexpr (BITS == 32) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[q] = __uint_as_float(w.code[q]);
+        return;
+    } else if constexpr (BITS == 16) {
         out[0] = __uint_as_float(w.code[0] << 16);
         out[1] = __uint_as_float(w.code[0] & 0xffff0000u);
-        out[2] = __uint_as_float(w.code[BITS == 16 ? 1 : 0] << 16);
-        out[3] = __uint_as_float(w.code[BITS == 16 ? 1 : 0] & 0xffff0000u);
+        out[2] = __uint_as_float(w.code[1] << 16);
+        out[3] = __uint_as_float(w.code[1] & 0xffff0000u);
         return;
     }
     const uint32_t c = w.code[0];
@@ -148,8 +162,9 @@ __global__ void __launch_bounds__(256, 2) k_project_batch(ProjectArgs a) {
     const int b = lane >> 2, i = lane & 3;
     const int r0 = blockIdx.x * 16 + wave * 4, t0 = blockIdx.y * T;
     const int steps = a.cols >> 6, row = min(r0 + i, a.rows - 1);
-    const uint8_t *row_codes = a.codes + (int64_t)row * a.cols * BITS / 8;
-    const int64_t row_groups = BITS == 16 ? 0 : (int64_t)row * (a.cols >> a.group_shift);
+    const bool gate = BITS == 32 && a.gate_row && row == a.rows - 1;
+    const uint8_t *row_codes = gate ? (const uint8_t *)a.gate_row : a.codes + (int64_t)row * a.cols * BITS / 8;
+    const int64_t row_groups = BITS >= 16 ? 0 : (int64_t)row * (a.cols >> a.group_shift);
     const float *row_scales = a.scales + row_groups, *row_offsets = (a.has_offset ? a.offsets : a.scales) + row_groups;
     // Each wave brings every fourth token's chunk: 256 columns, 1 KiB, one DMA.
     auto stage = [&](int c, int buf) {
@@ -226,9 +241,16 @@ __global__ void __launch_bounds__(256, 2) k_project_batch(ProjectArgs a) {
     const int quarter = lane >> 4, token = quarter == 1 ? 2 : quarter == 2 ? 1 : quarter;
 #pragma unroll
     for (int g = 0; g < NG; g++) {
-        const float y = tree_columns(acc[g]);
+        float y = tree_columns(acc[g]);
         const int t = t0 + 4 * g + token;
-        if ((lane & 15) < 4 && r0 + i < a.rows && t < a.tokens) a.Y[(int64_t)t * a.stride + a.out + r0 + i] = y;
+        if ((lane & 15) < 4 && r0 + i < a.rows && t < a.tokens) {
+            if (gate) {
+                a.gate_out[t] = y;
+            } else {
+                if (BITS == 32 && a.expert_bias) y = y + a.expert_bias[r0 + i];
+                a.Y[(int64_t)t * a.stride + a.out + r0 + i] = y;
+            }
+        }
     }
 }
 
@@ -324,6 +346,28 @@ void launch(sm_ctx *ctx, const ProjectArgs &a, int ng) {
     }
 }
 
+// Groups of tokens per wave. More of them share a weight's load and
+// widening, fewer make more blocks. Measured at 2,560 columns, a block
+// takes 8 / 10 / 17 us (1 / 2 / 4 groups) where every CU has one, and
+// 5 / 5 / 7 us for each further one a CU has to take; the least of those
+// sums is taken. bf16, in us with 1 / 2 / 4 groups: 10,240 rows x 4
+// tokens 17 / 20 / 31, x 16 54 / 31 / 31, x 32 105 / 58 / 49; 2,560 rows
+// x 12 12 / 14 / 17, x 16 18 / 14 / 17, x 32 28 / 20 / 23; 600 rows x 16
+// 10.5 / 10.7 / 17.
+int token_groups(int rows, int tokens) {
+    const int first[3] = {8, 10, 17}, further[3] = {5, 5, 7};
+    int ng = 1, best = 0;
+    for (int k = 0; k < 3; k++) {
+        const int64_t blocks = (int64_t)((rows + 15) / 16) * ((tokens + (4 << k) - 1) / (4 << k));
+        const int cost = first[k] + further[k] * (int)std::min<int64_t>((blocks - 1) / 256, 1 << 20);
+        if (k == 0 || cost < best) {
+            ng = 1 << k;
+            best = cost;
+        }
+    }
+    return ng;
+}
+
 }  // namespace
 
 namespace smi {
@@ -338,32 +382,27 @@ bool project_batch_takes(int bits, int cols, int tokens, uint64_t X, uint64_t co
 int project_batch(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets,
                   float *Y, int cols, int rows, int tokens, int stride, int out, int group, int bias, int codebook,
                   int has_offset) {
-    ProjectArgs a = {X, (const uint8_t *)codes, scales, offsets, Y, cols, rows, tokens, stride, out, 0, has_offset, (float)bias};
+    ProjectArgs a = {X, (const uint8_t *)codes, scales, offsets, Y, cols, rows, tokens, stride, out, 0, has_offset, (float)bias, nullptr, nullptr, nullptr};
     while (bits != 16 && (1 << a.group_shift) < group) a.group_shift++;
-    // Groups of tokens per wave. More of them share a weight's load and
-    // widening, fewer make more blocks. Measured at 2,560 columns, a block
-    // takes 8 / 10 / 17 us (1 / 2 / 4 groups) where every CU has one, and
-    // 5 / 5 / 7 us for each further one a CU has to take; the least of those
-    // sums is taken. bf16, in us with 1 / 2 / 4 groups: 10,240 rows x 4
-    // tokens 17 / 20 / 31, x 16 54 / 31 / 31, x 32 105 / 58 / 49; 2,560 rows
-    // x 12 12 / 14 / 17, x 16 18 / 14 / 17, x 32 28 / 20 / 23; 600 rows x 16
-    // 10.5 / 10.7 / 17.
-    const int first[3] = {8, 10, 17}, further[3] = {5, 5, 7};
-    int ng = 1, best = 0;
-    for (int k = 0; k < 3; k++) {
-        const int64_t blocks = (int64_t)((rows + 15) / 16) * ((tokens + (4 << k) - 1) / (4 << k));
-        const int cost = first[k] + further[k] * (int)std::min<int64_t>((blocks - 1) / 256, 1 << 20);
-        if (k == 0 || cost < best) {
-            ng = 1 << k;
-            best = cost;
-        }
-    }
+    const int ng = token_groups(rows, tokens);
     switch (bits) {
         case 2: launch<2, false>(ctx, a, ng); break;
         case 4: codebook == 1 ? launch<4, true>(ctx, a, ng) : launch<4, false>(ctx, a, ng); break;
         case 8: launch<8, false>(ctx, a, ng); break;
         default: launch<16, false>(ctx, a, ng); break;
     }
+    return launched(ctx);
+}
+
+bool route_batch_takes(const float *X, int width, const float *Wr, const float *gate_w) {
+    return width % 64 == 0 && ((uintptr_t)X | (uintptr_t)Wr | (uintptr_t)gate_w) % 16 == 0;
+}
+
+int route_batch(sm_ctx *ctx, const float *X, int tokens, int width, const float *Wr, const float *bias, int experts,
+                float *logits, const float *gate_w, float *gate_out) {
+    const ProjectArgs a = {X, (const uint8_t *)Wr, nullptr, nullptr, logits, width, experts + (gate_w ? 1 : 0), tokens, experts, 0,
+                           0, 0, 0.0f, gate_w, bias, gate_out};
+    launch<32, false>(ctx, a, token_groups(a.rows, tokens));
     return launched(ctx);
 }
 
@@ -381,7 +420,7 @@ bool project_one_takes(int bits, int cols, uint64_t X, uint64_t codes, uint64_t 
 
 int project_one(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets, float *Y,
                 int cols, int rows, int group, int bias, int codebook, int has_offset) {
-    ProjectArgs a = {X, (const uint8_t *)codes, scales, offsets, Y, cols, rows, 1, rows, 0, 0, has_offset, (float)bias};
+    ProjectArgs a = {X, (const uint8_t *)codes, scales, offsets, Y, cols, rows, 1, rows, 0, 0, has_offset, (float)bias, nullptr, nullptr, nullptr};
     while ((1 << a.group_shift) < group) a.group_shift++;
     int waves = 4;
     while (one_token_lds(bits, cols, group, waves) > kOneTokenLds) waves--;
