@@ -444,14 +444,28 @@ struct Ring<64> {
         return S == 0 ? g_big0 : S == 1 ? g_big1 : g_big2;
     }
 };
+// 16-row tiles (k_moe_gemm_stream16): 8 KiB stages, six of them (48 KiB,
+// three blocks per CU).
+__shared__ __attribute__((aligned(16))) RingStage<16> g_tiny0, g_tiny1, g_tiny2, g_tiny3, g_tiny4, g_tiny5;
+template <>
+struct Ring<16> {
+    static constexpr int NS = 6;
+    template <int S>
+    static __device__ __forceinline__ RingStage<16> &stage() {
+        return S == 0 ? g_tiny0 : S == 1 ? g_tiny1 : S == 2 ? g_tiny2 : S == 3 ? g_tiny3 : S == 4 ? g_tiny4 : g_tiny5;
+    }
+};
 // Calls f(stage S) for the S equal to `slot` (slot is a constant once the
 // group loop is unrolled).
 template <int BM, typename F>
 __device__ __forceinline__ void with_stage(int slot, F &&f) {
     switch (slot) {
     case 0: f(Ring<BM>::template stage<0>()); break;
-    case 1: f(Ring<BM>::template stage<1>()); break;
-    default: f(Ring<BM>::template stage<2>()); break;
+    case 1: f(Ring<BM>::template stage<1 % Ring<BM>::NS>()); break;
+    case 2: f(Ring<BM>::template stage<2 % Ring<BM>::NS>()); break;
+    case 3: f(Ring<BM>::template stage<3 % Ring<BM>::NS>()); break;
+    case 4: f(Ring<BM>::template stage<4 % Ring<BM>::NS>()); break;
+    default: f(Ring<BM>::template stage<5 % Ring<BM>::NS>()); break;
     }
 }
 
@@ -874,6 +888,297 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
         }
 }
 
+// ---------------------------------------------------------------------------
+// Batches of up to kStepTokens tokens, a decode step's, run through a stack of
+// layers, and there a product rounded elsewhere travels on: over 40 inputs,
+// four blocks of 32 tokens whose expert products differ in rounding alone end
+// up to 2e-5 apart. Their bits stay what they are: the two kernels below scale
+// the weights (k_moe_gemm_rows16 would take 74 instead of 77 us a block).
+//
+// k_moe_gemm_step16: k_moe_gemm_rows16's loads, with the four lane quarters of
+// one MFMA on four different groups and the scales on the weights.
+template <int NT>
+__device__ __forceinline__ void pin_scaled(v4u (&b)[NT], uint32_t (&s)[NT]) {
+#pragma unroll
+    for (int i = 0; i < NT; i++) asm volatile("" : "+v"(b[i]), "+v"(s[i]));
+}
+template <bool GATE_UP, int KG, int NT>
+__global__ void __launch_bounds__(256, 3) k_moe_gemm_step16(const _Float16 *__restrict__ A, const int *__restrict__ rows,
+                                                         const int4 *__restrict__ info, const int *__restrict__ tiles,
+                                                         const uint8_t *__restrict__ arena, uint64_t stride,
+                                                         const uint8_t *__restrict__ shared_blob, int experts,
+                                                         uint64_t codes_off, uint64_t scales_off, int K, int N,
+                                                         void *__restrict__ out, int out_ld) {
+    constexpr int BN = 64 * NT, G = KG, NSS = KG / 4;
+    static_assert(KG % 4 == 0 && KG >= 8 && KG <= STREAM_MAX_G, "whole supersteps of four groups");
+    static_assert(NT == 1 || NT == 2 || NT == 4, "1, 2 or 4 column tiles per wave");
+    (void)K;
+    (void)N;
+    int tau, cb;
+    xcd_tile(tau, cb);
+    if (tau >= tiles[experts + 1]) return;
+    const int4 ti = info[tau];
+    const int e = ti.x, m0 = ti.y, mend = ti.z;
+    const uint8_t *blob = e < experts ? arena + (uint64_t)e * stride : shared_blob;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = cb * BN, col = lane & 15, kq = lane >> 4;
+
+    // Activation DMA: chunk tid of a group is hi/lo tid / 128, row
+    // (tid / 8) % 16, slot tid % 8 holding part slot ^ ((row / 2) & 7).
+    const _Float16 *asrc;
+    {
+        const int hl = tid >> 7, r = (tid >> 3) & 15, part = (tid & 7) ^ ((r >> 1) & 7);
+        const int pos = min(m0 + r, mend - 1);  // rows past the end load the segment's last row
+        const int64_t arow = GATE_UP ? (e < experts ? rows[pos] : pos - ti.w) : pos;
+        asrc = A + (arow * G * 2 + hl) * 64 + part * 8;
+    }
+    // Group j of superstep S goes to 256 j of the superstep's half.
+    auto issue_a = [&](v4u *half, int S) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) dma16(asrc + (int64_t)(4 * S + j) * 128, &half[256 * j + 64 * wave]);
+    };
+    // Byte offsets from the block's blob (32 bits: a blob is under 4 GiB),
+    // so the loads take the blob address from scalar registers.
+    const uint8_t *bcodes = blob + codes_off, *bscales = blob + scales_off;
+    uint32_t boff[NT], soff[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) {
+        const uint32_t n = (uint32_t)(n0 + wave * 16 * NT + nt * 16 + col);
+        boff[nt] = n * (G * 16) + kq * 16;
+        soff[nt] = n * (G * 2) + kq * 2;
+    }
+    auto load_b = [&](v4u (&b)[NT], int S) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) b[nt] = *(const v4u *)(bcodes + boff[nt] + S * 64);
+    };
+    auto load_s = [&](uint32_t (&s)[NT], int S) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) s[nt] = *(const uint16_t *)(bscales + soff[nt] + S * 8);
+    };
+
+    const PairMagic magic = pair_magic();
+    float4v acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) acc[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+    auto compute = [&](const v4u *half, const v4u (&b)[NT], const uint32_t (&s)[NT]) {
+        half2v scale[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)s[nt]);
+            scale[nt] = (half2v){sh, sh};
+        }
+        const v4u *ag = half + 256 * kq;  // the lane's group of the superstep
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const int slot = t ^ ((col >> 1) & 7);
+            const half8 ahi = __builtin_bit_cast(half8, ag[col * 8 + slot]);
+            const half8 alo = __builtin_bit_cast(half8, ag[(16 + col) * 8 + slot]);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const uint32_t w = (t >> 1) == 0 ? b[nt].x : (t >> 1) == 1 ? b[nt].y : (t >> 1) == 2 ? b[nt].z : b[nt].w;
+                const half8 bb = b_operand_word(w >> (8 * (t & 1)), magic, scale[nt]);
+                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bb, acc[nt], 0, 0, 0);
+                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb, acc[nt], 0, 0, 0);
+            }
+        }
+    };
+    // Superstep S in flight: 4 DMAs, NT code loads, NT scale loads per
+    // thread, issued in that order, all of S before any of S + 1 (memory
+    // fences between the supersteps: the waits count loads in issue order).
+    // Three slots: superstep S + 2 is issued into the slot of S - 1 once
+    // every wave has passed the barrier that starts S.
+    constexpr int PER_SS = 4 + 2 * NT;
+    v4u b0[NT], b1[NT], b2[NT];
+    uint32_t s0[NT], s1[NT], s2[NT];
+    auto issue = [&](int S) {
+        if (S % 3 == 0) {
+            issue_a(g_rows16_0, S);
+            load_b(b0, S);
+            load_s(s0, S);
+        } else if (S % 3 == 1) {
+            issue_a(g_rows16_1, S);
+            load_b(b1, S);
+            load_s(s1, S);
+        } else {
+            issue_a(g_rows16_2, S);
+            load_b(b2, S);
+            load_s(s2, S);
+        }
+        asm volatile("" ::: "memory");
+    };
+    issue(0);
+    if (NSS > 1) issue(1);
+#pragma clang loop unroll(full)
+    for (int S = 0; S < NSS; S++) {
+        // Superstep S complete for this wave (S + 1 may stay in flight),
+        // then for every wave.
+        if (S + 1 < NSS) ring_sync<PER_SS>();
+        else ring_sync<0>();
+        if (S + 2 < NSS) issue(S + 2);
+        // The unpacking of the superstep's codes stays behind the wait (the
+        // compiler would otherwise start it early and wait for every load).
+        if (S % 3 == 0) {
+            pin_scaled(b0, s0);
+            compute(g_rows16_0, b0, s0);
+        } else if (S % 3 == 1) {
+            pin_scaled(b1, s1);
+            compute(g_rows16_1, b1, s1);
+        } else {
+            pin_scaled(b2, s2);
+            compute(g_rows16_2, b2, s2);
+        }
+    }
+
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int pos = m0 + 4 * kq + i, n = n0 + wave * 16 * NT + nt * 16 + col;
+            if (GATE_UP) {
+                const float other = sm::dpp_f32<sm::kDppQuadXor1>(acc[nt][i], acc[nt][i]);
+                if ((col & 1) == 0 && pos < mend) {
+                    const float h = silu_fast(acc[nt][i]) * other;
+                    const int jj = n >> 1;
+                    _Float16 *dst =
+                        (_Float16 *)out + ((int64_t)pos * (out_ld / 64) + (jj >> 6)) * 128 + k_position(jj & 63);
+                    const _Float16 hi = (_Float16)h;
+                    dst[0] = hi;
+                    dst[64] = (_Float16)(h - (float)hi);
+                }
+            } else if (pos < mend) {
+                ((float *)out)[(int64_t)pos * out_ld + n] = acc[nt][i];
+            }
+        }
+}
+
+// The streaming kernel for short segments: 16-row tiles on
+// v_mfma_f32_16x16x32_f16, so a segment of ~10 rows (the typical expert at a
+// few hundred tokens) pays for 16 rows of MFMA work instead of 32. Block:
+// 16 rows x 256 weight rows, 4 waves side by side in N, each 16 x 64 (four
+// 16 x 16 tiles). The 16x16x32 operands: lane l holds row (or column) l % 16
+// and K positions 8 (l / 16) .. +7 of a 32-wide step. With the K order of the
+// activations, step s of a 64-wide group and lane quarter kq = l / 16 map to
+// code word 2s + kq / 2, byte half kq % 2 (the same unpacking as the 32-row
+// kernel's lane halves) and to the 16-byte part 4s + kq of the A row.
+// Result: lane l holds rows 4 (l / 16) + i (i = 0..3) of column l % 16.
+template <bool GATE_UP, int KG>
+__global__ void __launch_bounds__(256) k_moe_gemm_stream16(const _Float16 *__restrict__ A, const int *__restrict__ rows,
+                                                           const int4 *__restrict__ info,
+                                                           const int *__restrict__ tiles,
+                                                           const uint8_t *__restrict__ arena, uint64_t stride,
+                                                           const uint8_t *__restrict__ shared_blob, int experts,
+                                                           uint64_t codes_off, uint64_t scales_off, int K, int N,
+                                                           void *__restrict__ out, int out_ld) {
+    constexpr int BM = 16, BN = 256, NT = 4;  // NT tiles of 16 columns per wave
+    using Stage = RingStage<BM>;
+    constexpr int NS = Ring<BM>::NS;
+    constexpr int G = KG;  // K / 64
+    static_assert(KG >= 8 && KG <= STREAM_MAX_G && KG % 2 == 0, "K / 64 groups");
+    (void)K;
+    (void)N;
+    // Tile record (segment, first row, end of the segment) from the dispatch.
+    int tau, cb;
+    xcd_tile(tau, cb);
+    if (tau >= tiles[experts + 1]) return;
+    const int4 ti = info[tau];
+    const int e = ti.x, m0 = ti.y, mend = ti.z;
+    const uint8_t *blob = e < experts ? arena + (uint64_t)e * stride : shared_blob;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = cb * BN;
+
+    // DMA sources, one A and one B load per thread per stage. A chunk
+    // c = tid: hi/lo c / 128, row (c / 8) % 16, slot c % 8 holding part
+    // slot ^ ((row / 2) & 7).
+    const _Float16 *asrc;
+    {
+        const int hl = tid >> 7, r = (tid >> 3) & 15, part = (tid & 7) ^ ((r >> 1) & 7);
+        const int pos = min(m0 + r, mend - 1);  // rows past the end load the segment's last row
+        const int64_t arow = GATE_UP ? (e < experts ? rows[pos] : pos - ti.w) : pos;
+        asrc = A + (arow * G * 2 + hl) * 64 + part * 8;
+    }
+    const uint8_t *bsrc = blob + codes_off + (uint64_t)(n0 + tid) * (G * 16);
+    auto issue = [&](Stage &sg, int g) {
+        dma16(asrc + (int64_t)g * 128, &sg.a[64 * wave]);
+        dma16(bsrc + (uint64_t)g * 16, &sg.b[64 * wave]);
+    };
+    const int col = lane & 15, kq = lane >> 4;
+    // Scales of the lane's four weight rows, every group, in registers.
+    uint32_t sreg[NT][G / 2];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+        load_row_scales<G>(blob + scales_off + (uint64_t)(n0 + wave * 64 + nt * 16 + col) * G * 2, sreg[nt]);
+#pragma clang loop unroll(full)
+    for (int q = 0; q < NS - 1; q++) with_stage<BM>(q, [&](Stage &sg) { issue(sg, min(q, G - 1)); });
+
+    const PairMagic magic = pair_magic();
+    // Byte selector of the lane's code word: word x (kq < 2) or y, moved
+    // down by one byte for odd kq (v_perm_b32: 0-3 pick bytes of the second
+    // source, 4-7 of the first, 0x0c gives zero).
+    const uint32_t psel = kq == 0 ? 0x03020100u : kq == 1 ? 0x0c030201u : kq == 2 ? 0x07060504u : 0x0c070605u;
+    float4v acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) acc[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+
+    auto compute = [&](const Stage &sg, int g) {
+        uint32_t words[NT][2];  // the lane's code word of step 0 and 1, shifted
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const v4u cv = sg.b[wave * 64 + nt * 16 + col];
+            words[nt][0] = __builtin_amdgcn_perm(cv.y, cv.x, psel);
+            words[nt][1] = __builtin_amdgcn_perm(cv.w, cv.z, psel);
+        }
+        half2v scale[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) {
+            const uint16_t s16 = (uint16_t)(sreg[nt][g >> 1] >> (16 * (g & 1)));
+            const _Float16 sh = __builtin_bit_cast(_Float16, s16);
+            scale[nt] = (half2v){sh, sh};
+        }
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const int part = 4 * s + kq, slot = part ^ ((col >> 1) & 7);
+            const half8 ahi = __builtin_bit_cast(half8, sg.a[col * 8 + slot]);
+            const half8 alo = __builtin_bit_cast(half8, sg.a[(BM + col) * 8 + slot]);
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                const half8 b = b_operand_word(words[nt][s], magic, scale[nt]);
+                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, b, acc[nt], 0, 0, 0);
+                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, b, acc[nt], 0, 0, 0);
+            }
+        }
+    };
+    constexpr int PS = 2;  // loads per thread per stage
+#pragma clang loop unroll(full)
+    for (int g = 0; g < G; g++) {
+        ring_sync<PS * (NS - 2)>();
+        with_stage<BM>((g + NS - 1) % NS, [&](Stage &sg) { issue(sg, min(g + NS - 1, G - 1)); });
+        with_stage<BM>(g % NS, [&](Stage &sg) { compute(sg, g); });
+    }
+    // No load may still be writing LDS when the block ends.
+    ring_sync<0>();
+
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int pos = m0 + 4 * kq + i, n = n0 + wave * 64 + nt * 16 + col;
+            if (GATE_UP) {
+                const float other = sm::dpp_f32<sm::kDppQuadXor1>(acc[nt][i], acc[nt][i]);
+                if ((col & 1) == 0 && pos < mend) {
+                    const float h = silu_fast(acc[nt][i]) * other;
+                    const int jj = n >> 1;
+                    _Float16 *dst =
+                        (_Float16 *)out + ((int64_t)pos * (out_ld / 64) + (jj >> 6)) * 128 + k_position(jj & 63);
+                    const _Float16 hi = (_Float16)h;
+                    dst[0] = hi;
+                    dst[64] = (_Float16)(h - (float)hi);
+                }
+            } else if (pos < mend) {
+                ((float *)out)[(int64_t)pos * out_ld + n] = acc[nt][i];
+            }
+        }
+}
+
 // Y[t, d] = P[shared(t), d] * sigmoid(gate[t]) + sum_k P[where[t,k], d] * w[t,k]
 // in the reference order (kernels/strata.cu:470-476); with `resid`,
 // Y = resid + that (strata_elementwise mode 5). One block per token (and
@@ -990,6 +1295,19 @@ StreamKernel small_kernel(bool gate_up, int groups, int small_nt) {
 }
 StreamKernel big_kernel(bool gate_up, int groups) { return small_kernel(gate_up, groups, 0); }
 
+// The products of up to kStepTokens tokens: 128 weight rows a block, or 256
+// with single groups (K = 640); null for other shapes.
+constexpr int kStepTokens = 64;
+StreamKernel step_kernel(bool gate_up, int groups) {
+    switch (groups) {
+        case 8: return gate_up ? k_moe_gemm_step16<true, 8, 2> : k_moe_gemm_step16<false, 8, 2>;
+        case 10: return gate_up ? k_moe_gemm_stream16<true, 10> : k_moe_gemm_stream16<false, 10>;
+        case 32: return gate_up ? k_moe_gemm_step16<true, 32, 2> : k_moe_gemm_step16<false, 32, 2>;
+        case 40: return gate_up ? k_moe_gemm_step16<true, 40, 2> : k_moe_gemm_step16<false, 40, 2>;
+        default: return nullptr;
+    }
+}
+
 struct PrefillWs {
     uint64_t logits, rcert, gate, dispatch, offsets, tiles_small, tiles_big, info_small, info_big,
         rows, parts, where_, Xhl, Hhl, P, Xn, end;
@@ -1047,8 +1365,11 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
     // rows in one 32-row tile, longer ones in 64-row tiles (k_moe_gemm).
     // (200 tokens at width 1,024, ff 256, 64 experts, top-6, the layer:
     // 125 us with k_moe_gemm, 46 us streaming.)
-    const bool stream = (2 * ff) % 256 == 0 && width % 256 == 0 && stream_groups(true, width / 64) &&
-                        stream_groups(false, ff / 64);
+    // Up to kStepTokens tokens: the four values of K that step_kernel has.
+    const bool step = tokens <= kStepTokens;
+    const bool stream = (2 * ff) % 256 == 0 && width % 256 == 0 &&
+                        (step ? step_kernel(true, width / 64) && step_kernel(false, ff / 64)
+                              : stream_groups(true, width / 64) && stream_groups(false, ff / 64));
     // Streaming shapes issue the split, the router and the dispatch on the
     // library's stream: a fork to the second stream and the join back inside
     // a graph cost more than the overlap they buy (A/B on one GPU, graph
@@ -1165,7 +1486,9 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
             }
             int rc_small = SM_OK;
             if (rc_big == SM_OK) {
-                small_kernel(gate_up, K / 64, small_nt)<<<dim3((unsigned)(N / (64 * small_nt)), small_tiles), 256, 0, ctx->stream>>>(
+                const auto ks = step ? step_kernel(gate_up, K / 64) : small_kernel(gate_up, K / 64, small_nt);
+                const int bn = step && K / 64 == 10 ? 256 : 64 * small_nt;  // weight rows per block
+                ks<<<dim3((unsigned)(N / bn), small_tiles), 256, 0, ctx->stream>>>(
                     a, r, info_small, tiles_small, ar, blob_stride, sh, experts, codes, scales, K, N, out, ld);
                 rc_small = launched(ctx);
             }
