@@ -36,6 +36,8 @@
 //    its tile record (segment, first row, end row, segment start) written by
 //    the dispatch, which tiles the shared expert's segment (every token) with
 //    the routed ones.
+//    Up to 64 tokens only the benchmark's and the real model's shapes stream,
+//    on kernels of their own (kStepTokens).
 //    Other shapes use k_moe_gemm (register-held B, A double-buffered in LDS,
 //    64- and 32-row tiles).
 //    grid.x = n-block (fastest) so the m-tiles of one (expert, n-block) run
@@ -1402,7 +1404,7 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
     const _Float16 *xhl = (const _Float16 *)(ws + w.Xhl), *hhl = (const _Float16 *)(ws + w.Hhl);
     const uint8_t *ar = (const uint8_t *)arena, *sh = (const uint8_t *)shared_blob;
 
-    // 16-row tiles: 256 weight rows per block, or 128 up to kSmallBatch tokens.
+    // Column tiles per wave of the 16-row kernels.
     const int small_nt = tokens <= kSmallBatch ? kSmallBatchColumnTiles : 4;
 
     // Other shapes: the split on the second stream, beside the router.
