@@ -232,7 +232,8 @@ int norm_launch(sm_ctx *ctx, const float *X, const float *gamma, float *Y, int c
 
 // Dense projections of a token batch (project_batch.hip), bit-identical to
 // the general kernels: bits 16 = bf16 weights, else quantized codes.
-bool project_batch_takes(int bits, int cols, int tokens, uint64_t X, uint64_t codes, int group, int bias, int codebook);
+bool project_batch_takes(int bits, int cols, int rows, int tokens, uint64_t X, uint64_t codes, int group, int bias,
+                         int codebook);
 int project_batch(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets,
                   float *Y, int cols, int rows, int tokens, int stride, int out, int group, int bias, int codebook,
                   int has_offset);

@@ -599,7 +599,7 @@ int L_quant_project(sm_ctx *ctx, const uint32_t *G, Args a) {
     if (int rc = need(ctx, a.ptr(2), (elems / groupSize) * 4, "Scales")) return rc;
     if (hasOffset)
         if (int rc = need(ctx, a.ptr(3), (elems / groupSize) * 4, "Offsets")) return rc;
-    if (project_batch_takes(bits, cols, tt, a.ptr(0), a.ptr(1), groupSize, bias, codebook))
+    if (project_batch_takes(bits, cols, rr, tt, a.ptr(0), a.ptr(1), groupSize, bias, codebook))
         return project_batch(ctx, bits, (const float *)a.ptr(0), (const void *)a.ptr(1), (const float *)a.ptr(2),
                              (const float *)a.ptr(3), (float *)a.ptr(4), cols, rr, tt, stride, off, groupSize, bias,
                              codebook, hasOffset != 0);
@@ -627,7 +627,7 @@ int L_bf16_project(sm_ctx *ctx, const uint32_t *G, Args a) {
             (const float *)a.ptr(0), (const uint32_t *)a.ptr(1), (float *)a.ptr(2), cols, rr, off);
         return launched(ctx);
     }
-    if (project_batch_takes(16, cols, tt, a.ptr(0), a.ptr(1), 0, 0, 0))
+    if (project_batch_takes(16, cols, rr, tt, a.ptr(0), a.ptr(1), 0, 0, 0))
         return project_batch(ctx, 16, (const float *)a.ptr(0), (const void *)a.ptr(1), nullptr, nullptr,
                              (float *)a.ptr(2), cols, rr, tt, stride, off, 0, 0, 0, 0);
     uint64_t total = (uint64_t)G[0] * G[1];

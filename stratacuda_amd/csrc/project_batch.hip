@@ -372,8 +372,15 @@ int token_groups(int rows, int tokens) {
 
 namespace smi {
 
-bool project_batch_takes(int bits, int cols, int tokens, uint64_t X, uint64_t codes, int group, int bias, int codebook) {
-    if (tokens < 2 || cols % 64 || X % 16 || codes % 8) return false;
+// Fewer outputs leave the batch kernel's blocks to a chain of load latencies,
+// which one wave per output beats (four matrices of 3,072 columns, us, batch
+// kernel against general: 600 outputs bf16 42 / 28, 4 bits 50 / 41; 1,500 bf16
+// 42 / 38; 2,400 43 / 42; 6,000 bf16 53 / 60, 4 bits 51 / 92).
+constexpr int64_t kBatchMinOutputs = 2560;
+
+bool project_batch_takes(int bits, int cols, int rows, int tokens, uint64_t X, uint64_t codes, int group, int bias,
+                         int codebook) {
+    if (tokens < 2 || (int64_t)rows * tokens < kBatchMinOutputs || cols % 64 || X % 16 || codes % 8) return false;
     if (bits == 16) return true;
     if (group < 4 || (group & (group - 1)) || (codebook == 1 && bits != 4)) return false;
     return bias > -(1 << 23) && bias < (1 << 23) - 256;

@@ -8,9 +8,9 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # cols, rows, tokens
-    (64, 1, 2), (64, 17, 33), (128, 15, 3), (192, 16, 4), (320, 65, 5), (704, 300, 8), (640, 33, 9), (2560, 4100, 16),
-    (3072, 50, 17), (1216, 8200, 32), (100, 20, 6)]
+SHAPES = [  # cols, rows, tokens; the first and the last take the general kernel (few outputs, ragged columns)
+    (64, 1, 2), (64, 1281, 2), (64, 97, 33), (128, 863, 3), (192, 640, 4), (320, 515, 5), (704, 337, 8), (640, 289, 9),
+    (2560, 4100, 16), (3072, 161, 17), (1216, 8200, 32), (100, 600, 6)]
 
 
 def same(a, b):
