@@ -752,15 +752,12 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
     // The group's products are summed over whole codes c - 1 and its scale,
     // one per column and so one per lane, goes on in f32.
     //
-    // PACK: a tile of up to eight rows puts their hi halves in rows 0-7 of the A
-    // operand and their lo halves in rows 8-15, one MFMA for both; the two are
-    // added at the end. For the batches whose experts mostly hold that few
-    // (the narrow tiles'); with four column tiles the second path costs more
-    // registers and code than it saves (512 tokens 196 -> 225 us).
-    constexpr bool PACK = NT == 2;
-    const bool packed = PACK && mend - m0 <= 8;
-    const int arow = packed ? col & 7 : col;
-    const int first = (packed ? (col >> 3) * 16 + arow : arow) * 8, second = (16 + arow) * 8;
+    // Every 16-row tile of every batch adds its products in this order, so a
+    // row's bits depend neither on its tile nor on NT. (Tiles of up to eight
+    // rows with hi and lo halves in one MFMA, the two sums added at the end,
+    // gained 5 to 9 % at 512 experts and up to 300 tokens; two equal tokens of
+    // a call then differed, and with the sums apart in all tiles every other
+    // batch lost 3 to 5 %.)
     auto compute = [&](const v4u *half, const v4u (&b)[NT], const v2u (&s)[NT], int S) {
         v4u words[NT];
 #pragma unroll
@@ -770,30 +767,19 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
             if (j >= groups_of(S)) break;
             const v4u *ag = half + 256 * j;
             float4v sum[NT];
-            half8 bb[2][NT];
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) sum[nt] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
-            auto part = [&](int at, int t) { return __builtin_bit_cast(half8, ag[at + ((2 * kq + t) ^ ((arow >> 1) & 7))]); };
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                const half8 ahi = part(first, t);
-                half8 alo;
-                if (!PACK) alo = part(second, t);
+                const int slot = (2 * kq + t) ^ ((col >> 1) & 7);
+                const half8 ahi = __builtin_bit_cast(half8, ag[col * 8 + slot]);
+                const half8 alo = __builtin_bit_cast(half8, ag[(16 + col) * 8 + slot]);
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++) {
                     const uint32_t w = j == 0 ? words[nt].x : j == 1 ? words[nt].y : j == 2 ? words[nt].z : words[nt].w;
-                    bb[t][nt] = b_codes_word(w >> (8 * t), magic);
-                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bb[t][nt], sum[nt], 0, 0, 0);
-                    if (!PACK) sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb[t][nt], sum[nt], 0, 0, 0);
-                }
-            }
-            if (PACK && !packed) {
-#pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    const half8 alo = part(second, t);
-#pragma unroll
-                    for (int nt = 0; nt < NT; nt++)
-                        sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bb[t][nt], sum[nt], 0, 0, 0);
+                    const half8 b8 = b_codes_word(w >> (8 * t), magic);
+                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, b8, sum[nt], 0, 0, 0);
+                    sum[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, b8, sum[nt], 0, 0, 0);
                 }
             }
 #pragma unroll
@@ -856,22 +842,10 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
         }
     }
 
-    // Packed: row r's hi sum is in lane quarter r / 4, its lo sum two quarters on.
-    if (packed) {
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const auto lo = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[nt][i]), __float_as_uint(acc[nt][i]),
-                                                                 false, false);
-                acc[nt][i] = acc[nt][i] + __uint_as_float(lo[1]);
-            }
-    }
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            // (packed: the quarters past row 7 fall past the segment's end)
             const int pos = m0 + 4 * kq + i, n = n0 + wave * 16 * NT + nt * 16 + col;
             if (GATE_UP) {
                 const float other = sm::dpp_f32<sm::kDppQuadXor1>(acc[nt][i], acc[nt][i]);
@@ -1251,10 +1225,11 @@ inline uint64_t up(uint64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 // 0.465 ms.)
 constexpr int kOneGridTokens = 1024;
 // Column tiles per wave of the 16-row kernel: two up to kSmallBatch tokens,
-// where the few tiles would leave CUs idle and most hold up to eight rows
-// (packed tiles), four above. Four against two, us a layer: 65 tokens 128.3 /
-// 122.8, 128 161 / 156, 200 177 / 174, 333 at 2560 / 640 288 / 282, 512 196 /
-// 199.
+// where the few tiles would leave CUs idle, four above. Four against two, us a
+// layer, at 65, 200 and 384 tokens: 512 experts top-10 at 2048 / 512 134 / 141,
+// 183 / 188 and 222 / 218, at 2560 / 640 218 / 207, 279 / 275 and 322 / 317;
+// 64 experts top-6 at 2048 / 512 64 / 55, 72 / 69 and 101 / 93, at 1024 / 256
+// 37 / 35, 43 / 41 and 53 / 51.
 constexpr int kSmallBatch = 384;
 constexpr int kSmallBatchColumnTiles = 2;
 inline int tiling_split(int tokens) { return tokens < kOneGridTokens ? tokens + 1 : 33; }

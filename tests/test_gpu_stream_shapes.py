@@ -42,3 +42,23 @@ def test_layer_group_counts(backend, oracle, W, F, E, topk, tokens, block):
     assert weights_ok(tokens, backend.read(w), ew)
     got, want = backend.read(Y), x + eY if block else eY
     assert tol_ok(got, want), "max abs err %g" % np.abs(got - want).max()
+
+
+@pytest.mark.parametrize("W,F,E,topk", [(1024, 256, 64, 6), (512, 384, 24, 3), (2560, 640, 12, 2), (2048, 512, 64, 6)])
+def test_equal_tokens_equal_results(backend, W, F, E, topk):
+    """Equal tokens get equal bits in every 16-row tile, the full ones and the
+    last one of 1 or 8 rows (of the shared segment, at least), and in calls of
+    up to 384 tokens and of more."""
+    layer = wl.DeviceLayer(backend, layer=0, width=W, ff=F, experts=E, base_seed=31)
+    rows = []
+    for tokens in (65, 200, 385):  # (from 512 tokens the weights come from the certified router)
+        x = backend.read(device_inputs(backend, tokens, W, 43, False)).reshape(tokens, W).copy()
+        x[-20:] = x[1]  # (the same values for every token count)
+        X, Y = backend.alloc(x.reshape(-1)), backend.alloc(tokens * W)
+        ids, w = backend.alloc(tokens * topk, "i32"), backend.alloc(tokens * topk)
+        ws = backend.alloc_bytes(backend.moe_workspace_bytes(tokens, W, F, E, topk))
+        backend.moe_layer(X, tokens, layer.Wr, layer.arena, layer.stride, layer.shared, layer.Wsg, W, F, E, topk, Y, ids, w, ws)
+        rows.append(backend.read(Y).view(np.uint32).reshape(tokens, W)[-20:])
+    layer.free()
+    rows = np.concatenate(rows)
+    assert np.array_equal(rows, np.broadcast_to(rows[0], rows.shape))
