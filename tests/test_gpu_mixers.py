@@ -18,7 +18,12 @@ def same(a, b):
 
 @pytest.mark.parametrize("dim,heads,kvh,position,tokens", [(256, 15, 3, 61, 20), (256, 24, 2, 1000, 11),
                                                            (128, 6, 2, 0, 1), (64, 5, 1, 63, 2), (128, 40, 2, 127, 25),
-                                                           (64, 34, 2, 190, 30), (256, 24, 2, 2047, 1)])
+                                                           (64, 34, 2, 190, 30), (256, 24, 2, 2047, 1),
+                                                           # one, two and three launches, and both kernels of scores
+                                                           (64, 32, 1, 60, 8), (64, 32, 1, 61, 8), (128, 17, 1, 8, 8), (128, 32, 1, 9, 8),
+                                                           (64, 8, 2, 632, 8), (64, 8, 2, 633, 8), (64, 32, 8, 700, 24), (64, 12, 1, 3, 5),
+                                                           (64, 32, 2, 40, 3), (128, 8, 2, 376, 8), (128, 8, 2, 377, 8), (128, 5, 1, 100, 7),
+                                                           (256, 3, 3, 381, 3), (256, 8, 2, 382, 3), (256, 24, 2, 58, 16), (256, 24, 2, 59, 16)])
 def test_attention_batch_edges(backend, oracle, dim, heads, kvh, position, tokens):
     rng = np.random.default_rng(dim + position)
     cells = position + tokens
