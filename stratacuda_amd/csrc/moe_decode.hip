@@ -1732,11 +1732,14 @@ int moe_decode(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias, 
             return rc;
     if (stage_on(ctx, kStageDecodeGateUp)) {
         if (int rc = stage_mark(ctx, kStageDecodeGateUp)) return rc;
-        // Twice the rows per wave once the grid has two blocks a CU without:
+        // Twice the rows per wave once the grid has three blocks a CU without:
         // four stack blocks of 4 tokens 133 -> 121 us, 5 162 -> 153, 6 179 ->
-        // 170, 2 at 2560 / 640 152 -> 136; a smaller grid loses (3 tokens of a
-        // 256-row expert, 336 blocks, 71 -> 73). Four times: 128, 150, 176, 137.
-        const int reps = (int64_t)blocks_per_expert * (topk + 1) * tokens <= 512 ? 1 : 2;
+        // 170, 2 at 2560 / 640 (880 blocks) 152 -> 136. A smaller grid loses:
+        // a layer's time without, divided by its time with, at widths 512 to
+        // 2304, ff 256 to 1536 and 1 to 6 tokens is 0.88 to 1.03 at 513 to 600
+        // blocks, 0.90 to 1.01 up to 700, 0.95 to 1.04 up to 800 and 0.97 to
+        // 1.10 up to 1,000. Four times the rows: 128, 150, 176, 137.
+        const int reps = (int64_t)blocks_per_expert * (topk + 1) * tokens <= 800 ? 1 : 2;
         dim3 g1((unsigned)ceil_div(blocks_per_expert, reps), (unsigned)(topk + 1), (unsigned)tokens);
         const int G = width / 64;
         const bool extra = G > 32 && G <= 40;
