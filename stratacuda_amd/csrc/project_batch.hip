@@ -373,14 +373,17 @@ int token_groups(int rows, int tokens) {
 namespace smi {
 
 // Fewer outputs leave the batch kernel's blocks to a chain of load latencies,
-// which one wave per output beats (four matrices of 3,072 columns, us, batch
-// kernel against general: 600 outputs bf16 42 / 28, 4 bits 50 / 41; 1,500 bf16
-// 42 / 38; 2,400 43 / 42; 6,000 bf16 53 / 60, 4 bits 51 / 92).
-constexpr int64_t kBatchMinOutputs = 2560;
+// which the general kernels' wave per output beats. Measured from graphs, three
+// matrices in turn, general over batch: bf16, 64 to 12,288 columns and 2 to 64
+// tokens, 0.62 to 0.99 at 2,600 outputs, 0.65 to 1.02 at 3,000, 0.81 to 1.13 at
+// 3,800, 0.92 to 1.25 at 4,200 and 1.02 to 1.42 at 5,400. The quantized general
+// kernels do more per weight: 1.00 to 1.66 at 2,600 to 2,900 outputs (fewer
+// were not measured over these ranges).
+int64_t batch_min_outputs(int bits) { return bits == 16 ? 4096 : 2560; }
 
 bool project_batch_takes(int bits, int cols, int rows, int tokens, uint64_t X, uint64_t codes, int group, int bias,
                          int codebook) {
-    if (tokens < 2 || (int64_t)rows * tokens < kBatchMinOutputs || cols % 64 || X % 16 || codes % 8) return false;
+    if (tokens < 2 || (int64_t)rows * tokens < batch_min_outputs(bits) || cols % 64 || X % 16 || codes % 8) return false;
     if (bits == 16) return true;
     if (group < 4 || (group & (group - 1)) || (codebook == 1 && bits != 4)) return false;
     return bias > -(1 << 23) && bias < (1 << 23) - 256;

@@ -1,16 +1,24 @@
 """Dense projections of a token batch on the GPU against the CPU oracle, bit for
 bit: strata_bf16_project and strata_quant_project at the edges of the batch
-kernel's tiles (4 weight rows a wave and 16 a block, groups of 4 tokens up to
-32, chunks of 4 x 64 columns and what is left of them) and, at one column count
-that is no multiple of 64, of the general kernel."""
+kernel's tiles (4 weight rows a wave and 16 a block, one, two and four groups of
+4 tokens a wave and what is left of them, chunks of 4 x 64 columns and what is
+left of them) and of the general kernels (few outputs, and one column count that
+is no multiple of 64)."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # cols, rows, tokens; the first and the last take the general kernel (few outputs, ragged columns)
+SHAPES = [  # cols, rows, tokens
+    # the general kernel for bf16 (few outputs), the first and the last for quantized weights too (few outputs, ragged columns)
     (64, 1, 2), (64, 1281, 2), (64, 97, 33), (128, 863, 3), (192, 640, 4), (320, 515, 5), (704, 337, 8), (640, 289, 9),
-    (2560, 4100, 16), (3072, 161, 17), (1216, 8200, 32), (100, 600, 6)]
+    (3072, 161, 17), (100, 600, 6),
+    # one group of tokens a wave
+    (64, 2305, 2), (64, 141, 33), (128, 1537, 3), (192, 1153, 4), (320, 923, 5), (640, 513, 9), (5120, 700, 7),
+    # two: 7, 13 of 16, 27 of 32 and all tokens; 1, 1, 2 and no steps past the last whole chunk
+    (64, 10240, 7), (320, 4100, 13), (128, 4100, 27), (2560, 4100, 16),
+    # four: 61 of 64, 30 of 32 and all; 3, 2 and 3 steps
+    (704, 2570, 61), (384, 6000, 30), (1216, 8200, 32)]
 
 
 def same(a, b):
