@@ -72,12 +72,17 @@ __global__ void __launch_bounds__(64) k_route_rows(const float *__restrict__ X, 
 // Tiles of TT tokens x TR rows per wave: 8 x 8 for large batches, 4 x 4 (four
 // times the waves) for small ones.
 constexpr int kRouteSmallTileMaxTokens = 128;
-// Fewer 8 x 8 tiles than two waves a SIMD run as a batched projection
-// (route_batch), whose blocks share the tokens' columns: layer of 200 tokens,
-// 512 experts 182 -> 176 us, 64 experts at width 1,024 44.6 -> 38.7. With more
-// the tiles win (300 tokens at 2,560 287 against 293 us, 500 at 2,048 227
-// against 235), as the 4 x 4 ones do (9 tokens, 47.7 against 49.6 us a block).
-constexpr int kRouteTileMinWaves = 2048;
+// Above, a batched projection (route_batch), which reads the router's weights
+// once for up to 16 tokens, while it has few blocks of 16 rows and 8 tokens;
+// then 8 x 8 tiles. Alone, with the weights in the L2s: tiles over projection,
+// widths 256 to 4,096, 1.0 to 1.7 up to 512 blocks (64 experts x 130 tokens at
+// 2,560 20.9 / 13.1 us, 256 x 200 21.3 / 19.7), from 513 to 1,000 0.81 to 1.11
+// (256 x 300 22.2 / 25.5, 512 x 130 21.6 / 25.3). In a layer (gate_w), where
+// the experts' weights have pushed them out, 512 experts, skewed: 561 to 660
+// blocks 1.01 to 1.04 (140 tokens at 2,048 89.9 / 86.5 us, at 2,560 117.7 /
+// 114.3), 825 to 990 0.96 to 1.00. The 4 x 4 tiles beat it too (9 tokens, 47.7
+// against 49.6 us a block).
+constexpr int kRouteBatchMaxBlocks = 512, kRouteBatchMaxBlocksLayer = 704;
 
 // One level of the reference's tree (lanes l and l ^ D added) over the N
 // outputs each lane still holds; lanes with bit D set keep the upper half.
@@ -583,7 +588,9 @@ int route_launch(sm_ctx *ctx, const float *X, int tokens, int width, const float
         const dim3 grid((unsigned)ceil_div(ceil_div(nrows, 4), 4), (unsigned)ceil_div(tokens, 4));
         k_route_gemm<4, 4><<<grid, 256, 0, ctx->stream>>>(X, Wr, bias, gate_w, logits, gate_out, tokens, width,
                                                           experts, gate_w ? 1 : 0);
-    } else if (ceil_div(nrows, 8) * ceil_div(tokens, 8) < kRouteTileMinWaves && route_batch_takes(X, width, Wr, gate_w)) {
+    } else if ((int64_t)ceil_div(nrows, 16) * ceil_div(tokens, 8) <=
+                   (gate_w ? kRouteBatchMaxBlocksLayer : kRouteBatchMaxBlocks) &&
+               route_batch_takes(X, width, Wr, gate_w)) {
         if (int rc = route_batch(ctx, X, tokens, width, Wr, bias, experts, logits, gate_w, gate_out)) return rc;
     } else {
         const dim3 grid((unsigned)ceil_div(ceil_div(nrows, 8), 4), (unsigned)ceil_div(tokens, 8));

@@ -100,3 +100,19 @@ def test_quant_one_token(backend, oracle, cols, rows, nbits, group, codebook, of
     got = backend.read(y)
     same(got[:rows], np.asarray(want, np.float32).reshape(-1)[:rows])
     assert got[rows] == -7
+
+
+@pytest.mark.parametrize("W,E,tokens", [(320, 64, 300), (384, 40, 129), (192, 256, 253), (192, 256, 257), (2560, 8, 131)])
+def test_route_batch(backend, oracle, W, E, tokens):
+    """The router by the batched projection: one group of tokens a wave (131 and
+    129 tokens), two with 4 and 5 of 8 tokens left, and past its last size the tiles."""
+    rng = np.random.default_rng(W + tokens)
+    x, wr = rng.normal(0, 1, tokens * W).astype(np.float32), rng.normal(0, 0.05, E * W).astype(np.float32)
+    bias, K = rng.normal(0, 1, E).astype(np.float32), 5
+    logits, ids, w = backend.alloc(tokens * E), backend.alloc(tokens * K, "i32"), backend.alloc(tokens * K)
+    backend.moe_route(backend.alloc(x), tokens, W, backend.alloc(wr), E, K, ids, w, logits=logits, bias=backend.alloc(bias))
+    want = (oracle.project(x, wr, W, E, tokens).reshape(tokens, E) + bias).reshape(-1)
+    same(backend.read(logits), want)
+    rids, rw = oracle.router(want, E, K, tokens)
+    assert np.array_equal(backend.read(ids), rids)
+    same(backend.read(w), rw)
