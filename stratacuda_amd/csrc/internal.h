@@ -242,8 +242,8 @@ bool route_batch_takes(const float *X, int width, const float *Wr, const float *
 int route_batch(sm_ctx *ctx, const float *X, int tokens, int width, const float *Wr, const float *bias, int experts,
                 float *logits, const float *gate_w, float *gate_out);
 // The same of one token, quantized codes only (strata_quant_gemv).
-bool project_one_takes(int bits, int cols, uint64_t X, uint64_t codes, uint64_t scales, uint64_t offsets, int group, int bias,
-                       int codebook);
+bool project_one_takes(int bits, int cols, int rows, uint64_t X, uint64_t codes, uint64_t scales, uint64_t offsets, int group,
+                       int bias, int codebook);
 int project_one(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets, float *Y,
                 int cols, int rows, int group, int bias, int codebook, int has_offset);
 

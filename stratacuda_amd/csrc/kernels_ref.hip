@@ -653,7 +653,7 @@ int L_quant_gemv(sm_ctx *ctx, const uint32_t *G, Args a) {
     if (int rc = need(ctx, a.ptr(2), (elems / groupSize) * 4, "Scales")) return rc;
     if (hasOffset)
         if (int rc = need(ctx, a.ptr(3), (elems / groupSize) * 4, "Offsets")) return rc;
-    if (project_one_takes(bits, cols, a.ptr(0), a.ptr(1), a.ptr(2), hasOffset ? a.ptr(3) : 0, groupSize, bias, codebook))
+    if (project_one_takes(bits, cols, rr, a.ptr(0), a.ptr(1), a.ptr(2), hasOffset ? a.ptr(3) : 0, groupSize, bias, codebook))
         return project_one(ctx, bits, (const float *)a.ptr(0), (const void *)a.ptr(1), (const float *)a.ptr(2),
                            (const float *)a.ptr(3), (float *)a.ptr(4), cols, rr, groupSize, bias, codebook, hasOffset != 0);
     k_quant_project<<<blocks_for(G[0]), 256, 0, ctx->stream>>>(

@@ -91,6 +91,24 @@ __device__ __forceinline__ void load_raw(const ProjectArgs &a, const uint8_t *ro
     }
 }
 
+// The values of four quantized weights, before their scale and offset.
+template <int BITS, bool CODEBOOK>
+__device__ __forceinline__ void unpack(const ProjectArgs &a, uint32_t c, float (&out)[4]) {
+    if (CODEBOOK) {
+        // the four codes in four bytes, looked up in the table's two halves
+        const uint32_t t = (c | c << 8) & 0x00ff00ffu, b = (t | t << 4) & 0x0f0f0f0fu, s = b & 0x07070707u;
+        const uint32_t lo = __builtin_amdgcn_perm(iq4_word(-49, -35, -22, -10), iq4_word(-127, -104, -83, -65), s);
+        const uint32_t hi = __builtin_amdgcn_perm(iq4_word(53, 69, 89, 113), iq4_word(1, 13, 25, 38), s);
+        const uint32_t m = ((b >> 3) & 0x01010101u) * 255u, v = (hi & m) | (lo & ~m);
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[q] = (float)((int)(v << (24 - 8 * q)) >> 24);
+    } else {
+        // code + bias: both are whole numbers below 2^23, so the f32 sum is exact
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[q] = (float)((c >> (BITS * q)) & ((1u << BITS) - 1u)) + a.bias;
+    }
+}
+
 // Widens the four weights in the reference's steps (kernels/strata.cu:168-211).
 // Without offsets +0 is added: that can only turn a weight of -0 into +0, and
 // no partial sum tells a product of -0 from one of +0.
@@ -106,26 +124,14 @@ __device__ __forceinline__ void widen(const ProjectArgs &a, const Raw<BITS> &w, 
         out[2] = __uint_as_float(w.code[1] << 16);
         out[3] = __uint_as_float(w.code[1] & 0xffff0000u);
         return;
-    }
-    const uint32_t c = w.code[0];
-    if (CODEBOOK) {
-        // the four codes in four bytes, looked up in the table's two halves
-        const uint32_t t = (c | c << 8) & 0x00ff00ffu, b = (t | t << 4) & 0x0f0f0f0fu, s = b & 0x07070707u;
-        const uint32_t lo = __builtin_amdgcn_perm(iq4_word(-49, -35, -22, -10), iq4_word(-127, -104, -83, -65), s);
-        const uint32_t hi = __builtin_amdgcn_perm(iq4_word(53, 69, 89, 113), iq4_word(1, 13, 25, 38), s);
-        const uint32_t m = ((b >> 3) & 0x01010101u) * 255u, v = (hi & m) | (lo & ~m);
-#pragma unroll
-        for (int q = 0; q < 4; q++) out[q] = (float)((int)(v << (24 - 8 * q)) >> 24);
     } else {
-        // code + bias: both are whole numbers below 2^23, so the f32 sum is exact
+        unpack<BITS, CODEBOOK>(a, w.code[0], out);
 #pragma unroll
-        for (int q = 0; q < 4; q++) out[q] = (float)((c >> (BITS * q)) & ((1u << BITS) - 1u)) + a.bias;
+        for (int q = 0; q < 4; q++) out[q] = out[q] * w.scale;
+        const float offset = a.has_offset ? w.offset : 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[q] = out[q] + offset;
     }
-#pragma unroll
-    for (int q = 0; q < 4; q++) out[q] = out[q] * w.scale;
-    const float offset = a.has_offset ? w.offset : 0.0f;
-#pragma unroll
-    for (int q = 0; q < 4; q++) out[q] = out[q] + offset;
 }
 
 // The reference's tree over columns for one group's 4 x 4 products: partial
@@ -265,65 +271,108 @@ __global__ void __launch_bounds__(256, 2) k_project_batch(ProjectArgs a) {
 // instructions (seven a weight) and the stream about equally. 2,560 x 10,240
 // with 32-weight groups and offsets, from a graph, us: 4 bits 13.7 -> 10.4, 8
 // bits 20.1 -> 14.6; 3,072 x 300 at 8 bits 11.2 -> 7.7.
+//
+// PIECES: rows whose LDS leaves a CU few waves come in pieces of 1,024 or 2,048
+// columns, the sums going on from one to the next. FINE: groups of one and two
+// weights, a scale a column.
 constexpr uint64_t kOneTokenLds = 65536;
 __host__ __device__ constexpr int one_token_pitch(int bits, int cols) {
     const int words = cols * bits / 32;
     return words + (2 * bits + 32 - words % 32) % 32;
 }
-template <int BITS, bool CODEBOOK>
+// Groups of a row, or those that a piece of it holds or lies in (group sizes are powers of two).
+__host__ __device__ constexpr int one_token_groups(int piece, int shift) { return (piece >> shift) > 0 ? piece >> shift : 1; }
+enum OneToken { WHOLE, FINE, PIECES };
+template <int BITS, bool CODEBOOK, OneToken MODE>
 __global__ void __launch_bounds__(256) k_project_one(ProjectArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint32_t s_one[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    const int b = lane >> 2, i = lane & 3, steps = a.cols >> 6;
-    const int words = a.cols * BITS / 32, pitch = one_token_pitch(BITS, a.cols), ng = a.cols >> a.group_shift;
+    const int b = lane >> 2, i = lane & 3, piece = MODE == PIECES ? a.tokens : a.cols;  // (one token: its slot holds the piece)
+    const int row_words = a.cols * BITS / 32, row_groups = a.cols >> a.group_shift;
+    const int pitch = one_token_pitch(BITS, piece), ng = MODE == PIECES ? one_token_groups(piece, a.group_shift) : row_groups;
     float *s_x = (float *)s_one;
-    uint32_t *codes = s_one + a.cols + wave * 4 * (pitch + 2 * ng);
+    uint32_t *codes = s_one + piece + wave * 4 * (pitch + 2 * ng);
     float *scales = (float *)(codes + 4 * pitch), *offsets = scales + 4 * ng;
     const int r0 = (blockIdx.x * waves + wave) * 4, nr = min(4, a.rows - r0);
-    for (int c = 256 * wave; c < a.cols; c += 256 * waves)
-        if (c + 4 * lane < a.cols)
-            __builtin_amdgcn_global_load_lds(a.X + c + 4 * lane, (lds_void_t *)(s_x + c), 16, 0, 0);
-    for (int r = 0; r < nr; r++) {
-        const uint8_t *row = a.codes + (int64_t)(r0 + r) * words * 4;
-        for (int c = 0; c < words; c += 256)
-            if (c + 4 * lane < words)
-                __builtin_amdgcn_global_load_lds(row + 4 * (c + 4 * lane), (lds_void_t *)(codes + r * pitch + c), 16, 0, 0);
-    }
-    // (four rows' groups are whole 16-byte pieces, fewer rows' may not be)
-    auto groups = [&](const float *src, float *dst) {
-        src += (int64_t)r0 * ng;
-        if (nr == 4) {
-            for (int c = 0; c < 4 * ng; c += 256)
-                if (c + 4 * lane < 4 * ng)
-                    __builtin_amdgcn_global_load_lds(src + c + 4 * lane, (lds_void_t *)(dst + c), 16, 0, 0);
-        } else {
-            for (int c = 0; c < nr * ng; c += 64)
-                if (c + lane < nr * ng) __builtin_amdgcn_global_load_lds(src + c + lane, (lds_void_t *)(dst + c), 4, 0, 0);
-        }
-    };
-    groups(a.scales, scales);
-    if (a.has_offset) groups(a.offsets, offsets);
-    __builtin_amdgcn_s_waitcnt(0 | 0x7 << 4 | 0xF << 8);  // vmcnt(0)
-    __syncthreads();
-    if (nr < 1) return;
-    const int row = min(i, nr - 1);
-    const uint8_t *code = (const uint8_t *)(codes + row * pitch) + b * BITS / 2;
-    const float *sc = scales + row * ng, *of = (a.has_offset ? offsets : scales) + row * ng, *x = s_x + 4 * b;
     float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 8
-    for (int k = 0; k < steps; k++) {
-        Raw<BITS> raw;
-        const uint8_t *c = code + k * 8 * BITS;
-        raw.code[0] = BITS == 8 ? *(const uint32_t *)c : BITS == 4 ? *(const uint16_t *)c : *c;
-        const int g = (64 * k + 4 * b) >> a.group_shift;
-        raw.scale = sc[g];
-        raw.offset = of[g];
-        const f32x4 xv = *(const f32x4 *)(x + 64 * k);
-        float w[4];
-        widen<BITS, CODEBOOK>(a, raw, w);
+    for (int p0 = 0; MODE != PIECES || p0 < a.cols; p0 += piece) {
+        const int n = MODE == PIECES ? min(piece, a.cols - p0) : a.cols, words = n * BITS / 32, g0 = p0 >> a.group_shift;
+        if (p0) __syncthreads();  // the last piece has been read
+        for (int c = 256 * wave; c < n; c += 256 * waves)
+            if (c + 4 * lane < n)
+                __builtin_amdgcn_global_load_lds(a.X + p0 + c + 4 * lane, (lds_void_t *)(s_x + c), 16, 0, 0);
+        for (int r = 0; r < nr; r++) {
+            const uint8_t *src = a.codes + ((int64_t)(r0 + r) * row_words + p0 * BITS / 32) * 4;
+            for (int c = 0; c < words; c += 256)
+                if (c + 4 * lane < words)
+                    __builtin_amdgcn_global_load_lds(src + 4 * (c + 4 * lane), (lds_void_t *)(codes + r * pitch + c), 16, 0, 0);
+        }
+        // (four rows' groups are whole 16-byte pieces, fewer rows' may not be;
+        // PIECES: one row's are if they are in every piece)
+        auto groups = [&](const float *src, float *dst) {
+            src += (int64_t)r0 * row_groups;
+            if constexpr (MODE == PIECES) {
+                const int ngp = ((p0 + n - 1) >> a.group_shift) - g0 + 1;
+                for (int r = 0; r < nr; r++) {
+                    const float *from = src + (int64_t)r * row_groups + g0;
+                    float *to = dst + r * ng;
+                    if (((row_groups | g0 | ngp | ng) & 3) == 0) {
+                        for (int c = 0; c < ngp; c += 256)
+                            if (c + 4 * lane < ngp)
+                                __builtin_amdgcn_global_load_lds(from + c + 4 * lane, (lds_void_t *)(to + c), 16, 0, 0);
+                    } else {
+                        for (int c = 0; c < ngp; c += 64)
+                            if (c + lane < ngp) __builtin_amdgcn_global_load_lds(from + c + lane, (lds_void_t *)(to + c), 4, 0, 0);
+                    }
+                }
+            } else if (nr == 4) {
+                for (int c = 0; c < 4 * ng; c += 256)
+                    if (c + 4 * lane < 4 * ng)
+                        __builtin_amdgcn_global_load_lds(src + c + 4 * lane, (lds_void_t *)(dst + c), 16, 0, 0);
+            } else {
+                for (int c = 0; c < nr * ng; c += 64)
+                    if (c + lane < nr * ng) __builtin_amdgcn_global_load_lds(src + c + lane, (lds_void_t *)(dst + c), 4, 0, 0);
+            }
+        };
+        groups(a.scales, scales);
+        if (a.has_offset) groups(a.offsets, offsets);
+        __builtin_amdgcn_s_waitcnt(0 | 0x7 << 4 | 0xF << 8);  // vmcnt(0)
+        __syncthreads();
+        if (nr < 1) {
+            if (MODE == PIECES) continue;
+            return;
+        }
+        const int row = min(i, nr - 1), steps = n >> 6;
+        const uint8_t *code = (const uint8_t *)(codes + row * pitch) + b * BITS / 2;
+        const float *sc = scales + row * ng, *of = (a.has_offset ? offsets : scales) + row * ng, *x = s_x + 4 * b;
+        constexpr int UNROLL = MODE == FINE ? 4 : 8;
+#pragma unroll UNROLL
+        for (int k = 0; k < steps; k++) {
+            Raw<BITS> raw;
+            const uint8_t *c = code + k * 8 * BITS;
+            raw.code[0] = BITS == 8 ? *(const uint32_t *)c : BITS == 4 ? *(const uint16_t *)c : *c;
+            const int col = p0 + 64 * k + 4 * b, g = (col >> a.group_shift) - g0;
+            const f32x4 xv = *(const f32x4 *)(x + 64 * k);
+            float w[4];
+            if constexpr (MODE == FINE) {
+                unpack<BITS, CODEBOOK>(a, raw.code[0], w);
 #pragma unroll
-        for (int q = 0; q < 4; q++) sum[q] = sum[q] + w[q] * xv[q];
+                for (int q = 0; q < 4; q++) {
+                    const int gq = (col + q) >> a.group_shift;
+                    w[q] = w[q] * sc[gq];
+                    w[q] = w[q] + (a.has_offset ? of[gq] : 0.0f);
+                }
+            } else {
+                raw.scale = sc[g];
+                raw.offset = of[g];
+                widen<BITS, CODEBOOK>(a, raw, w);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) sum[q] = sum[q] + w[q] * xv[q];
+        }
+        if constexpr (MODE != PIECES) break;
     }
+    if (MODE == PIECES && nr < 1) return;
     // the reference's tree: columns 32, 16, 8 and 4 apart are lanes, 2 and 1 are q
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -416,28 +465,65 @@ int route_batch(sm_ctx *ctx, const float *X, int tokens, int width, const float 
     return launched(ctx);
 }
 
-// LDS of a block of `waves` waves.
-static uint64_t one_token_lds(int bits, int cols, int group, int waves) {
-    return 4ull * (cols + (uint64_t)waves * 4 * (one_token_pitch(bits, cols) + 2 * (cols / group)));
+static int log2_of(int n) { return 31 - __builtin_clz((unsigned)n); }
+// LDS of a block of `waves` waves and pieces of `piece` columns; the most
+// waves that kOneTokenLds holds, and how many of them a CU does.
+static uint64_t one_token_lds(int bits, int piece, int shift, int waves) {
+    return 4ull * (piece + (uint64_t)waves * 4 * (one_token_pitch(bits, piece) + 2 * one_token_groups(piece, shift)));
+}
+static int one_token_waves(int bits, int piece, int shift) {
+    int waves = 4;
+    while (waves > 0 && one_token_lds(bits, piece, shift, waves) > kOneTokenLds) waves--;
+    return waves;
+}
+static int one_token_waves_per_cu(int bits, int piece, int shift) {
+    const int waves = one_token_waves(bits, piece, shift);
+    return waves ? waves * (int)(163840 / one_token_lds(bits, piece, shift, waves)) : 0;
 }
 
-bool project_one_takes(int bits, int cols, uint64_t X, uint64_t codes, uint64_t scales, uint64_t offsets, int group, int bias,
-                       int codebook) {
+bool project_one_takes(int bits, int cols, int rows, uint64_t X, uint64_t codes, uint64_t scales, uint64_t offsets, int group,
+                       int bias, int codebook) {
     if (cols % 64 || (X | codes | scales | offsets) % 16) return false;
-    if (group < 4 || (group & (group - 1)) || (codebook == 1 && bits != 4)) return false;
-    return bias > -(1 << 23) && bias < (1 << 23) - 256 && one_token_lds(bits, cols, group, 1) <= kOneTokenLds;
+    if ((group & (group - 1)) || (codebook == 1 && bits != 4)) return false;
+    // Groups of one and two weights, whose scales are most of a row: up to 256
+    // a row, and only with many rows (8 bits, general over this: 256 columns in
+    // groups of one 3.8 / 4.5 us at 300 rows, 4.8 / 4.6 at 3,072, 9.2 / 7.7 at
+    // 10,240).
+    if (group < 4 && (cols / group > 256 || rows <= 2048)) return false;
+    return bias > -(1 << 23) && bias < (1 << 23) - 256 && one_token_waves(bits, cols, log2_of(group)) > 0;
+}
+
+template <OneToken MODE>
+static auto one_token_kernel(int bits, int codebook) {
+    return bits == 2   ? k_project_one<2, false, MODE>
+           : bits == 8 ? k_project_one<8, false, MODE>
+                       : (codebook == 1 ? k_project_one<4, true, MODE> : k_project_one<4, false, MODE>);
 }
 
 int project_one(sm_ctx *ctx, int bits, const float *X, const void *codes, const float *scales, const float *offsets, float *Y,
                 int cols, int rows, int group, int bias, int codebook, int has_offset) {
-    ProjectArgs a = {X, (const uint8_t *)codes, scales, offsets, Y, cols, rows, 1, rows, 0, 0, has_offset, (float)bias, nullptr, nullptr, nullptr};
-    while ((1 << a.group_shift) < group) a.group_shift++;
-    int waves = 4;
-    while (one_token_lds(bits, cols, group, waves) > kOneTokenLds) waves--;
-    const auto k = bits == 2   ? k_project_one<2, false>
-                   : bits == 8 ? k_project_one<8, false>
-                               : (codebook == 1 ? k_project_one<4, true> : k_project_one<4, false>);
-    k<<<(unsigned)((rows + 4 * waves - 1) / (4 * waves)), 64 * waves, one_token_lds(bits, cols, group, waves), ctx->stream>>>(a);
+    // Pieces once whole rows leave a CU six waves or fewer, the rows fill the
+    // GPU more than once and pieces at least double the waves; the shorter ones
+    // where the longer leave fewer than twelve and more than one round. 10,240
+    // rows of 8 bits, whole / in pieces, us: 4,096 columns 35.8 / 20.6 with
+    // 16-weight groups (27.7 in the longer ones) and 26.8 / 19.4 with 32; 6,144
+    // columns 55.6 / 24.0; 2,100 rows of 4,096 9.3 / 9.6.
+    const int shift = log2_of(group), whole = one_token_waves_per_cu(bits, cols, shift);
+    int piece = cols;
+    if (cols >= 4096 && whole <= 6 && rows > 256 * 4 * whole)
+        for (int p : {2048, 1024}) {
+            const int per_cu = one_token_waves_per_cu(bits, p, shift);
+            if (per_cu >= 2 * whole) piece = p;
+            if (per_cu >= 12 || rows <= 256 * 4 * per_cu) break;
+        }
+    const bool pieces = piece < cols;
+    const int waves = one_token_waves(bits, piece, shift);
+    const ProjectArgs a = {X,  (const uint8_t *)codes, scales, offsets,    Y,          cols,    rows,    pieces ? piece : 1,
+                           rows, 0, shift, has_offset, (float)bias, nullptr, nullptr, nullptr};
+    const auto k = pieces      ? one_token_kernel<PIECES>(bits, codebook)
+                   : group < 4 ? one_token_kernel<FINE>(bits, codebook)
+                               : one_token_kernel<WHOLE>(bits, codebook);
+    k<<<(unsigned)((rows + 4 * waves - 1) / (4 * waves)), 64 * waves, one_token_lds(bits, piece, shift, waves), ctx->stream>>>(a);
     return launched(ctx);
 }
 

@@ -78,9 +78,15 @@ def test_quant_batch(backend, oracle, cols, rows, tokens, nbits, group, codebook
     same(backend.read(y), want)
 
 
-@pytest.mark.parametrize("cols,rows", [(64, 1), (128, 3), (320, 17), (2560, 4100), (4096, 66), (3072, 301), (100, 7)])
-@pytest.mark.parametrize("nbits,group,codebook,offset", [(4, 32, 0, 1), (8, 32, 0, 1), (4, 64, 1, 0), (2, 4, 0, 0),
-                                                         (8, 64, 0, 0), (2, 32, 0, 1), (4, 2, 0, 1)])
+ONE_TOKEN = [(cols, rows, *form) for cols, rows in ((64, 1), (128, 3), (320, 17), (2560, 4100), (4096, 66), (3072, 301), (100, 7))
+             for form in ((4, 32, 0, 1), (8, 32, 0, 1), (4, 64, 1, 0), (2, 4, 0, 0), (8, 64, 0, 0), (2, 32, 0, 1), (4, 2, 0, 1))]
+# groups of one and two weights, by the general kernel and (more than 2,048 rows, up to 256 groups each) from LDS;
+# rows in pieces of 2,048 columns (groups of 16 and 4, a group of two pieces, a short last piece of one group) and 1,024
+ONE_TOKEN += [(256, 35, 8, 1, 0, 1), (576, 2050, 8, 2, 0, 1), (256, 2051, 8, 1, 0, 1), (192, 2054, 2, 1, 0, 0), (512, 2049, 4, 2, 1, 1),
+              (4096, 3101, 8, 16, 0, 1), (4096, 2051, 4, 4, 1, 1), (8192, 3074, 4, 4096, 0, 1), (6208, 3079, 8, 64, 0, 0), (4096, 8195, 8, 16, 0, 1)]
+
+
+@pytest.mark.parametrize("cols,rows,nbits,group,codebook,offset", ONE_TOKEN)
 def test_quant_one_token(backend, oracle, cols, rows, nbits, group, codebook, offset):
     """One token: blocks of four, three and fewer waves (the rows' bytes in LDS), waves of four rows and fewer."""
     if cols % group:
