@@ -28,8 +28,9 @@
 //    shuffle; the activations are stored in the same order, so staging them
 //    into LDS is a plain 16-byte copy and the MFMA A operand one 16-byte read.
 //  * Tiles (width a multiple of 256 up to 2,560, ff of 128; stream_groups): below
-//    1,024 tokens every segment runs in 16 x 256 blocks on
-//    v_mfma_f32_16x16x32_f16 (k_moe_gemm_rows16), one grid; from 1,024 tokens
+//    1,024 tokens every segment runs in blocks of 16 x 128 (up to 384 tokens) or
+//    16 x 256 on v_mfma_f32_16x16x32_f16 (k_moe_gemm_rows16), one grid; from 1,024
+//    tokens
 //    segments of more than 32 rows run in 64 x 256 blocks on
 //    v_mfma_f32_32x32x16_f16 (k_moe_gemm_stream), the two grids covering
 //    disjoint rows and running on two streams. Each block reads
@@ -37,7 +38,7 @@
 //    the dispatch, which tiles the shared expert's segment (every token) with
 //    the routed ones.
 //    Up to 64 tokens only the benchmark's and the real model's shapes stream,
-//    on kernels of their own (kStepTokens).
+//    on kernels of their own (kStepTokens: k_moe_gemm_step16, k_moe_gemm_stream16).
 //    Other shapes use k_moe_gemm (register-held B, A double-buffered in LDS,
 //    64- and 32-row tiles).
 //    grid.x = n-block (fastest) so the m-tiles of one (expert, n-block) run
@@ -632,16 +633,14 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 // took 131 us at 333 tokens with a ring of single groups, 78 us so). Weight
 // codes go from HBM straight to the lanes that use them: in superstep S, lane
 // (col, kq) of wave w loads the 16 code bytes of group 4S + kq of weight rows
-// n0 + 64w + 16nt + col (nt = 0..3). One load
-// instruction then reads 64 contiguous bytes of each of 16 rows (reading 16
-// bytes of each of 64 rows instead, with the weights staged through LDS,
-// streams at about half the rate), and the lane holds exactly its B operands
-// of the superstep's eight 32-wide MFMA steps: step t takes word t / 2, byte
-// half t % 2 of its group. The four lane quarters of one MFMA thus work on
-// four different groups, with the activations read to match; the sum over K
-// is the same. Activations (16 rows x 4 groups, hi/lo, 16 KiB a superstep)
-// are staged in LDS by DMA, three slots deep: lane (row col, kq) reads part t
-// of group 4S + kq. One barrier per superstep.
+// n0 + 16 NT w + 16 nt + col (nt < NT). One load instruction then reads 64
+// contiguous bytes of each of 16 rows (reading 16 bytes of each of 64 rows
+// instead, with the weights staged through LDS, streams at about half the
+// rate). A 4 x 4 transpose between the lane quarters leaves quarter kq word kq
+// of every group, so that one MFMA works on one group: step t takes byte half
+// t of the word and part 2 kq + t of the activation row. Activations (16 rows
+// x 4 groups, hi/lo, 16 KiB a superstep) are staged in LDS by DMA, three slots
+// deep. One barrier per superstep.
 __shared__ __attribute__((aligned(16))) v4u g_rows16_0[4 * 256], g_rows16_1[4 * 256], g_rows16_2[4 * 256];
 
 // An empty volatile statement that reads and rewrites the registers: code
@@ -674,8 +673,8 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
                                                          const uint8_t *__restrict__ shared_blob, int experts,
                                                          uint64_t codes_off, uint64_t scales_off, int K, int N,
                                                          void *__restrict__ out, int out_ld) {
-    // NT column tiles of 16 per wave: a block covers 64 NT weight rows (NT = 4
-    // for most batches; 1 where few tiles would leave the GPU idle).
+    // NT column tiles of 16 per wave: a block covers 64 NT weight rows (see
+    // kSmallBatch).
     constexpr int BN = 64 * NT, G = KG, NSS = (KG + 3) / 4;
     constexpr bool HALF = KG % 4 == 2;  // the last superstep has two groups
     static_assert(KG % 2 == 0 && KG >= 2 && KG <= STREAM_MAX_G, "an even number of groups");
@@ -868,26 +867,31 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
 // Batches of up to kStepTokens tokens, a decode step's, run through a stack of
 // layers, and there a product rounded elsewhere travels on: over 40 inputs,
 // four blocks of 32 tokens whose expert products differ in rounding alone end
-// up to 2e-5 apart. Their bits stay what they are: the two kernels below scale
-// the weights (k_moe_gemm_rows16 would take 74 instead of 77 us a block).
+// up to 2e-5 apart. Their bits stay what they are, at a cost: the two kernels
+// below scale the weights (k_moe_gemm_rows16 took 74 instead of 77 us a block of
+// 32 tokens), and shapes without them run k_moe_gemm (64 tokens at width 1,024,
+// ff 256, 64 experts 123 us a block, where a layer of 65 takes 35).
 //
-// k_moe_gemm_step16: k_moe_gemm_rows16's loads, with the four lane quarters of
-// one MFMA on four different groups and the scales on the weights.
+// k_moe_gemm_step16: k_moe_gemm_rows16's loads without its transpose: lane (col,
+// kq) holds its B operands of the superstep's eight 32-wide MFMA steps as they
+// come, step t in word t / 2, byte half t % 2 of its group. The four lane
+// quarters of one MFMA thus work on four different groups, with the
+// activations read to match (part t of group 4S + kq) and the scales on the
+// weights; the sum over K is the same. Two column tiles a wave.
 template <int NT>
 __device__ __forceinline__ void pin_scaled(v4u (&b)[NT], uint32_t (&s)[NT]) {
 #pragma unroll
     for (int i = 0; i < NT; i++) asm volatile("" : "+v"(b[i]), "+v"(s[i]));
 }
-template <bool GATE_UP, int KG, int NT>
+template <bool GATE_UP, int KG>
 __global__ void __launch_bounds__(256, 3) k_moe_gemm_step16(const _Float16 *__restrict__ A, const int *__restrict__ rows,
                                                          const int4 *__restrict__ info, const int *__restrict__ tiles,
                                                          const uint8_t *__restrict__ arena, uint64_t stride,
                                                          const uint8_t *__restrict__ shared_blob, int experts,
                                                          uint64_t codes_off, uint64_t scales_off, int K, int N,
                                                          void *__restrict__ out, int out_ld) {
-    constexpr int BN = 64 * NT, G = KG, NSS = KG / 4;
+    constexpr int NT = 2, BN = 64 * NT, G = KG, NSS = KG / 4;
     static_assert(KG % 4 == 0 && KG >= 8 && KG <= STREAM_MAX_G, "whole supersteps of four groups");
-    static_assert(NT == 1 || NT == 2 || NT == 4, "1, 2 or 4 column tiles per wave");
     (void)K;
     (void)N;
     int tau, cb;
@@ -1027,17 +1031,17 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_step16(const _Float16 *__re
         }
 }
 
-// The streaming kernel for short segments: 16-row tiles on
-// v_mfma_f32_16x16x32_f16, so a segment of ~10 rows (the typical expert at a
-// few hundred tokens) pays for 16 rows of MFMA work instead of 32. Block:
-// 16 rows x 256 weight rows, 4 waves side by side in N, each 16 x 64 (four
-// 16 x 16 tiles). The 16x16x32 operands: lane l holds row (or column) l % 16
+// k_moe_gemm_stream16: the down product of K = 640 for these batches, whose
+// ten groups are no whole supersteps: 16-row tiles like the 64-row kernel's,
+// codes and activations in an LDS ring of single groups. Block: 16 rows x 256
+// weight rows, 4 waves side by side in N, each 16 x 64 (four 16 x 16 tiles).
+// The 16x16x32 operands: lane l holds row (or column) l % 16
 // and K positions 8 (l / 16) .. +7 of a 32-wide step. With the K order of the
 // activations, step s of a 64-wide group and lane quarter kq = l / 16 map to
 // code word 2s + kq / 2, byte half kq % 2 (the same unpacking as the 32-row
 // kernel's lane halves) and to the 16-byte part 4s + kq of the A row.
 // Result: lane l holds rows 4 (l / 16) + i (i = 0..3) of column l % 16.
-template <bool GATE_UP, int KG>
+template <int KG>
 __global__ void __launch_bounds__(256) k_moe_gemm_stream16(const _Float16 *__restrict__ A, const int *__restrict__ rows,
                                                            const int4 *__restrict__ info,
                                                            const int *__restrict__ tiles,
@@ -1052,6 +1056,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm_stream16(const _Float16 *__res
     static_assert(KG >= 8 && KG <= STREAM_MAX_G && KG % 2 == 0, "K / 64 groups");
     (void)K;
     (void)N;
+    (void)rows;
     // Tile record (segment, first row, end of the segment) from the dispatch.
     int tau, cb;
     xcd_tile(tau, cb);
@@ -1069,8 +1074,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm_stream16(const _Float16 *__res
     {
         const int hl = tid >> 7, r = (tid >> 3) & 15, part = (tid & 7) ^ ((r >> 1) & 7);
         const int pos = min(m0 + r, mend - 1);  // rows past the end load the segment's last row
-        const int64_t arow = GATE_UP ? (e < experts ? rows[pos] : pos - ti.w) : pos;
-        asrc = A + (arow * G * 2 + hl) * 64 + part * 8;
+        asrc = A + ((int64_t)pos * G * 2 + hl) * 64 + part * 8;
     }
     const uint8_t *bsrc = blob + codes_off + (uint64_t)(n0 + tid) * (G * 16);
     auto issue = [&](Stage &sg, int g) {
@@ -1138,20 +1142,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm_stream16(const _Float16 *__res
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int pos = m0 + 4 * kq + i, n = n0 + wave * 64 + nt * 16 + col;
-            if (GATE_UP) {
-                const float other = sm::dpp_f32<sm::kDppQuadXor1>(acc[nt][i], acc[nt][i]);
-                if ((col & 1) == 0 && pos < mend) {
-                    const float h = silu_fast(acc[nt][i]) * other;
-                    const int jj = n >> 1;
-                    _Float16 *dst =
-                        (_Float16 *)out + ((int64_t)pos * (out_ld / 64) + (jj >> 6)) * 128 + k_position(jj & 63);
-                    const _Float16 hi = (_Float16)h;
-                    dst[0] = hi;
-                    dst[64] = (_Float16)(h - (float)hi);
-                }
-            } else if (pos < mend) {
-                ((float *)out)[(int64_t)pos * out_ld + n] = acc[nt][i];
-            }
+            if (pos < mend) ((float *)out)[(int64_t)pos * out_ld + n] = acc[nt][i];
         }
 }
 
@@ -1277,10 +1268,10 @@ StreamKernel big_kernel(bool gate_up, int groups) { return small_kernel(gate_up,
 constexpr int kStepTokens = 64;
 StreamKernel step_kernel(bool gate_up, int groups) {
     switch (groups) {
-        case 8: return gate_up ? k_moe_gemm_step16<true, 8, 2> : k_moe_gemm_step16<false, 8, 2>;
-        case 10: return gate_up ? k_moe_gemm_stream16<true, 10> : k_moe_gemm_stream16<false, 10>;
-        case 32: return gate_up ? k_moe_gemm_step16<true, 32, 2> : k_moe_gemm_step16<false, 32, 2>;
-        case 40: return gate_up ? k_moe_gemm_step16<true, 40, 2> : k_moe_gemm_step16<false, 40, 2>;
+        case 8: return gate_up ? k_moe_gemm_step16<true, 8> : k_moe_gemm_step16<false, 8>;
+        case 10: return gate_up ? nullptr : k_moe_gemm_stream16<10>;  // (no width is 640: N is a multiple of 256)
+        case 32: return gate_up ? k_moe_gemm_step16<true, 32> : k_moe_gemm_step16<false, 32>;
+        case 40: return gate_up ? k_moe_gemm_step16<true, 40> : k_moe_gemm_step16<false, 40>;
         default: return nullptr;
     }
 }
@@ -1341,7 +1332,7 @@ int moe_prefill(sm_ctx *ctx, uint64_t X, int tokens, uint64_t Wr, uint64_t bias,
     // longer ones run in 64-row tiles. Other shapes: segments of up to 32
     // rows in one 32-row tile, longer ones in 64-row tiles (k_moe_gemm).
     // (200 tokens at width 1,024, ff 256, 64 experts, top-6, the layer:
-    // 125 us with k_moe_gemm, 46 us streaming.)
+    // 125 us with k_moe_gemm, 38 us streaming.)
     // Up to kStepTokens tokens: the four values of K that step_kernel has.
     const bool step = tokens <= kStepTokens;
     const bool stream = (2 * ff) % 256 == 0 && width % 256 == 0 &&
