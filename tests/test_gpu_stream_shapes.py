@@ -1,11 +1,10 @@
 """The prefill layer at the group counts of the streaming products against the
 CPU oracle: K / 64 of 4 .. 36 in the gate/up product, and in the down product
 one superstep of two groups (ff 128), whole ones, and whole ones with two more;
-up to 64 tokens (the kernels of a decode step's batches), up to 384 (128 weight
-rows a block, tiles of up to eight rows packed), up to 1,023 (256) and from
-1,024 (64-row tiles beside them). 129 to 511 tokens with few experts route by
-the batched projection. One shape past the streaming kernels' (width 384) takes
-the general ones."""
+up to 384 tokens (128 weight rows a block), up to 1,023 (256) and from 1,024
+(64-row tiles beside them). Up to 64 tokens these shapes take the general
+kernels, as one past the streaming kernels' (width 384) does at any count. 129
+to 511 tokens with few experts route by the batched projection."""
 import numpy as np
 import pytest
 
@@ -18,7 +17,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("W,F,E,topk,tokens", [(256, 128, 8, 3, 7), (256, 128, 40, 3, 65), (256, 128, 8, 3, 1030), (768, 384, 12, 4, 64),
                                                (1024, 256, 64, 6, 65), (1280, 896, 10, 2, 33), (1024, 640, 9, 3, 200), (1024, 640, 40, 3, 384), (512, 640, 9, 3, 385), (256, 128, 17, 2, 511),
-                                               (1792, 1024, 6, 2, 1024), (2304, 1280, 6, 2, 50), (384, 192, 8, 3, 90)])
+                                               (1792, 1024, 6, 2, 1024), (2304, 1280, 6, 2, 50), (384, 192, 8, 3, 90),
+                                               (768, 384, 12, 4, 65), (768, 384, 12, 4, 385), (768, 384, 12, 4, 1024), (1280, 896, 10, 2, 66),
+                                               (1280, 896, 10, 2, 390), (2304, 1280, 6, 2, 67), (2304, 1280, 6, 2, 386)])
 @pytest.mark.parametrize("block", [False, True])
 def test_layer_group_counts(backend, oracle, W, F, E, topk, tokens, block):
     layer = wl.DeviceLayer(backend, layer=0, width=W, ff=F, experts=E, base_seed=29)
