@@ -23,11 +23,12 @@
 // registers one chunk ahead.
 //
 // Bound: vector issue from about 8 tokens (16 tokens: 64 adds and 16 matrix
-// instructions a step; without its loads the kernel takes 26 of its 31 us),
-// the weights' stream below (a load's latency per chunk, 3 TB/s). bf16, 2,560
-// x 10,240 x 16 tokens: 208 -> 31 us, where one wave per output and token
-// read each weight 16 times. Three or four chunks of weights in registers
-// were slower (35 us: fewer waves fit and the loads past the end count).
+// instructions a step; vector instructions issue 57 % of the SIMDs' time, the
+// matrix unit is busy 15 %), the weights' stream below (a load's latency per
+// chunk, 3 TB/s). bf16, 2,560 x 10,240 x 16 tokens: 208 -> 33 us, where one
+// wave per output and token read each weight 16 times. Three or four chunks
+// of weights in registers were slower (35 against 31 us in one run: fewer
+// waves fit and the loads past the end count).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
