@@ -754,7 +754,7 @@ __global__ void __launch_bounds__(256, 3) k_moe_gemm_rows16(const _Float16 *__re
     // Every 16-row tile of every batch adds its products in this order, so a
     // row's bits depend neither on its tile nor on NT. (Tiles of up to eight
     // rows with hi and lo halves in one MFMA, the two sums added at the end,
-    // gained 5 to 9 % at 512 experts and up to 300 tokens; two equal tokens of
+    // gained 3 to 9 % at 512 experts and up to 300 tokens; two equal tokens of
     // a call then differed, and with the sums apart in all tiles every other
     // batch lost 3 to 5 %.)
     auto compute = [&](const v4u *half, const v4u (&b)[NT], const v2u (&s)[NT], int S) {
